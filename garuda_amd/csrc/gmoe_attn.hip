@@ -14,10 +14,10 @@
 // are tokens, each with its sequence's page table, its position and the position
 // attention starts at; entries of one sequence come in position order, so the append
 // kernel writes every entry's k and v before any attends (causal within the call).
+// Calls of several tokens of a sequence (prompts) run tiles of rows on MFMA (k_attn_tile).
 #include "gmoe_device.h"
 
 namespace gmoe {
-
 
 // simd::rope for pair i of a head at position pos: the frequency theta^(-2i/hd) and
 // the angle in f32 as the reference forms them.
@@ -97,6 +97,51 @@ __global__ void __launch_bounds__(256) k_rope_append(AttnArgs a) {
     vp[hoff + 2 * j] = vx;
     vp[hoff + 2 * j + 1] = vy;
   }
+}
+
+// k_rope_append for calls of many tokens, gridDim.y workgroups a token: a thread makes its
+// pair's angle once for every head it rotates (the powf and sincosf were most of the
+// launch), with up to kRopeHeads heads' loads issued before it. Copies the call's entries
+// and tiles to the device for the launches after it.
+constexpr uint32_t kRopeHeads = 8;
+__global__ void __launch_bounds__(256) k_rope_rows(AttnArgs a) {
+  const uint32_t i = blockIdx.x, t = threadIdx.x, half = a.hd / 2, ng = 256 / half, j = t % half, g = t / half;
+  const AttnEntry e = a.hent[i];
+  if (t == 0 && blockIdx.y == 0) {
+    const_cast<AttnEntry*>(a.ent)[i] = e;
+    if (i < a.ntile) const_cast<AttnTile*>(a.tiles)[i] = a.htile[i];
+  }
+  const uint32_t slot = e.pos % a.bs, kvd = a.n_kv * a.hd, nh = a.n_heads + a.n_kv, step = ng * gridDim.y;
+  if (e.fresh && t == 0 && blockIdx.y == 0) e.pages[e.pos / a.bs] = e.page;  // read by the attention kernel after this one
+  float* kp = a.pool + (size_t)e.page * a.page_floats + (size_t)slot * a.hd;  // head h at + h * bs * hd
+  float* vp = kp + (size_t)a.bs * kvd;
+  const float* vs = a.v + (size_t)i * a.kv_stride;
+  float x[kRopeHeads], y[kRopeHeads], cs = 0.0f, sn = 0.0f;
+  for (uint32_t h0 = g + ng * blockIdx.y; g < ng && h0 < nh; h0 += kRopeHeads * step) {
+#pragma unroll
+    for (uint32_t b = 0; b < kRopeHeads; b++) {
+      const uint32_t h = min(h0 + b * step, nh - 1);
+      const float* src = h < a.n_heads ? a.q + (size_t)i * a.q_stride + h * a.hd
+                                       : a.k + (size_t)i * a.kv_stride + (h - a.n_heads) * a.hd;
+      x[b] = src[2 * j];
+      y[b] = src[2 * j + 1];
+    }
+    if (h0 < step) {
+      const float freq = 1.0f / powf(a.theta, (2.0f * (float)j) / (float)a.hd);
+      sincosf((float)e.pos * freq, &sn, &cs);
+    }
+#pragma unroll
+    for (uint32_t b = 0; b < kRopeHeads; b++) {
+      const uint32_t h = h0 + b * step;
+      if (h < nh) {
+        float* dst = h < a.n_heads ? a.qr + ((size_t)i * a.n_heads + h) * a.hd : kp + (size_t)(h - a.n_heads) * a.bs * a.hd;
+        dst[2 * j] = x[b] * cs - y[b] * sn;
+        dst[2 * j + 1] = x[b] * sn + y[b] * cs;
+      }
+    }
+  }
+  for (uint32_t z = t + 256 * blockIdx.y; z < kvd; z += 256 * gridDim.y)
+    vp[(size_t)(z / a.hd) * a.bs * a.hd + z % a.hd] = vs[z];
 }
 
 __device__ __forceinline__ float wave_max(float v) { return wave64_max(v); }
@@ -355,6 +400,387 @@ __global__ void __launch_bounds__(256) k_attn_combine(AttnArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------------
+// Tiled attention: runs of tokens of one sequence (a prompt's positions).
+//
+// One workgroup per (kv head, tile of 256 (token, query head) rows, split of the keys), 8
+// waves of 32 rows. The single-token kernels read a kv head's keys and values once for
+// every token; here a 32-key tile in LDS serves 256 rows. The products run on bf16 MFMA at
+// f32 precision: an f32 is the sum of three bf16 of 8 bits each (split3, exact), and of
+// the nine products of two such sums the six down to 2^-16 of the first are taken; the
+// three left out are below 2^-23 of it, an f32 product's own rounding. Six passes of
+// v_mfma_f32_32x32x16_bf16 take 3/8 of the cycles of v_mfma_f32_32x32x2_f32.
+//   S^T = K Q^T: A = the keys (row l % 32), B = the wave's queries, so lane l holds the
+//     scores of query l % 32 for keys 8 (r / 4) + 4 (l / 32) + r % 4, r = 0..15;
+//   O^T = V^T P^T: with those keys taken in that order, lane l's own 16 probabilities are
+//     the B operand as they stand; A is V^T (row d = l % 32), transposed while staged.
+// So a row's softmax state sits in two lanes (l, l ^ 32), and no probability moves.
+// Grid x is the kv head: workgroups go round-robin over the 8 XCDs, so with 8 kv heads a
+// head's keys and values are read into one XCD's L2.
+//
+// Measured (a 1500-token prompt in 256-token calls, 32 heads on 8 of 128): 35 us a call on
+// average, against 198 us of k_attn_partial; its products are 5.9 GFLOP at 1400 keys, 35
+// GFLOP in six passes. A 32-key tile takes 3.9 us where its MFMAs take 2.6 (8 waves); 6 us
+// of a call are its start (tile, pages, first keys, queries) and its partial rows. With f32
+// MFMA instead the same call took 54 us. Row sums: the tile's products are summed by
+// themselves, smallest planes first, then added to the row's in one rounding (error against
+// 64 bits 1.7e-7; 3e-7 with one long chain, 1.9e-7 in the single-token kernels).
+//
+// Non-finite input: 0 * inf and inf - inf make NaNs of what f32 products would leave alone
+// (keys beside a row's span, -inf scores), so a row that meets a non-finite score or ends
+// with a non-finite sum is marked and summed by itself (attn_serial).
+// ---------------------------------------------------------------------------------
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+// x = a + b + c, the upper halves of the three words: 8 significant bits each.
+__device__ __forceinline__ void split3(float x, uint32_t& a, uint32_t& b, uint32_t& c) {
+  a = __float_as_uint(x);
+  const float r = x - __uint_as_float(a & 0xffff0000u);
+  b = __float_as_uint(r);
+  c = __float_as_uint(r - __uint_as_float(b & 0xffff0000u));
+}
+// The upper halves of lo and hi as a bf16 pair.
+__device__ __forceinline__ uint32_t bf_pair(uint32_t lo, uint32_t hi) {
+  return __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+}
+// N values (even) as three planes of bf16 pairs.
+template <int N>
+__device__ __forceinline__ void split_planes(const float* x, uint32_t (*w)[N / 2]) {
+#pragma unroll
+  for (int i = 0; i < N / 2; i++) {
+    uint32_t a0, b0, c0, a1, b1, c1;
+    split3(x[2 * i], a0, b0, c0);
+    split3(x[2 * i + 1], a1, b1, c1);
+    w[0][i] = bf_pair(a0, a1);
+    w[1][i] = bf_pair(b0, b1);
+    w[2][i] = bf_pair(c0, c1);
+  }
+}
+__device__ __forceinline__ bf16x8 frag4(const uint32_t* w) {
+  return __builtin_bit_cast(bf16x8, u32x4{w[0], w[1], w[2], w[3]});
+}
+__device__ __forceinline__ f32x16 mfma_bf(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+// c += the five smaller products of a * b, two values split in three planes.
+__device__ __forceinline__ f32x16 mfma_rest(const bf16x8* a, const bf16x8* b, f32x16 c) {
+  c = mfma_bf(a[2], b[0], c);
+  c = mfma_bf(a[0], b[2], c);
+  c = mfma_bf(a[1], b[1], c);
+  c = mfma_bf(a[1], b[0], c);
+  return mfma_bf(a[0], b[1], c);
+}
+
+// A split's max may be a mark: a row for attn_serial (a NaN pattern no max can be).
+constexpr uint32_t kMarkSerial = 0x7fc00001u;
+
+__device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 64); }
+
+template <int NT>  // head_dim = 32 NT
+__global__ void __launch_bounds__(512, 2) k_attn_tile(AttnArgs a) {
+  constexpr uint32_t HD = 32 * NT, KT = kAttnTileKeys, KS = HD / 16;
+  // a buffer: keys [plane][key][HD], 16-byte column x at x ^ (key % KX); values transposed
+  // [plane][d][KT] in rows of 80 bytes (which spread a column's 16-byte reads over all
+  // banks). Two buffers: the next tile is loaded while this one's products run (to LDS, a
+  // thread's own 16 bytes at a time: the registers are full), then split and written, with
+  // one barrier a tile.
+  constexpr uint32_t KX = NT == 4 ? 16 : NT == 2 ? 8 : 4, KPL = KT * HD * 2, VP = 2 * KT + 16, VPL = HD * VP;
+  constexpr uint32_t BUF = 3 * (KPL + VPL);
+  constexpr int NK = (NT + 1) / 2;  // key float4 a thread
+  static_assert(KT == 32 && kAttnTileRows == 256, "one MFMA row tile of keys, eight of rows");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * BUF];
+  __shared__ float4 raw[NK + 2 < 4 ? 2048 : (NK + 2) * 512];  // at least 4 KB a wave for the output
+  __shared__ uint32_t tab[2][KT];  // pool rows (of HD floats) of a tile's keys
+  const uint32_t h = blockIdx.x, c = blockIdx.z, tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hf = lane >> 5;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t G = a.n_heads / a.n_kv;
+  const AttnTile* T = a.tiles + blockIdx.y;
+  auto uni = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane(v); };
+  const uint32_t i0 = uni(T->i0), r0 = uni(T->r0), nr = uni(T->nr);
+  const uint32_t pos0 = uni(T->pos0), start1 = uni(T->start1);
+  const uint32_t k0 = uni(T->start0) + c * a.skeys, k1 = min(uni(T->pos1) + 1, k0 + a.skeys);
+  const uint32_t row = 32 * wave + l32, rr = r0 + min(row, nr - 1), i = i0 + rr / G;
+  const uint32_t head = h * G + rr % G, rows = a.n * a.n_heads;
+  const uint32_t prow = c * rows + i * a.n_heads + head;  // the row's partial
+  float* pml = a.part + (size_t)a.nchunk * rows * HD;
+  const bool mine = row < nr;
+  if (k0 >= k1) {  // past the tile's span: an empty split
+    if (mine && hf == 0) {
+      pml[2 * (size_t)prow] = -INFINITY;
+      pml[2 * (size_t)prow + 1] = 0.0f;
+    }
+    return;
+  }
+  const uint32_t pos = a.ent[i].pos, start = a.ent[i].start;
+  const uint32_t* pages = T->pages;
+  const uint32_t prows = 2 * a.bs * a.n_kv;  // pool rows of a page
+  // page and row in it of a key position (the product waits for the page's load)
+  auto look = [&](uint32_t p, uint32_t& page, uint32_t& off) {
+    const uint32_t q = min(p, k1 - 1), pg = q / a.bs;
+    page = pages[pg];
+    off = h * a.bs + (q - pg * a.bs);
+  };
+  if (tid < 2 * KT) {
+    uint32_t page, off;
+    look(k0 + tid, page, off);
+    tab[tid / KT][tid % KT] = page * prows + off;
+  }
+  f32x16 o[NT], zero;
+#pragma unroll
+  for (int r = 0; r < 16; r++) zero[r] = 0.0f;
+#pragma unroll
+  for (int t = 0; t < NT; t++) o[t] = zero;
+  float M = -INFINITY, L = 0.0f;  // M in units of log2, as the scores below
+  bool odd = false;               // a non-finite score was seen
+  const float sc2 = a.scale * 0x1.715476p+0f;  // log2 e
+  // staging: the thread's keys (float4 kx of keys it / (8 NT)), and of the values a pair of
+  // keys kp and four columns dq
+  const uint32_t kp = lane % 16, dq = 4 * wave + lane / 16;
+  const uint32_t vwo = 3 * KPL + 4 * dq * VP + 16 * (2 * (kp / 8) + (kp / 2) % 2) + 8 * ((kp / 4) % 2) + 4 * (kp % 2);
+  const bool vmine = wave < 2 * NT;
+  const float4* vpool = reinterpret_cast<const float4*>(a.pool + (size_t)a.bs * a.n_kv * HD);
+  auto load = [&](uint32_t b) {
+    auto lds16 = [&](const float4* src, uint32_t j) {
+      __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)(raw + 512 * j + 64 * wave), 16, 0, 0);
+    };
+#pragma unroll
+    for (int j = 0; j < NK; j++) {
+      const uint32_t it = j * 512 + tid, key = it / (8 * NT), x = it % (8 * NT);
+      if ((j + 1) * 512 <= 256 * NT || 64 * wave < 256 * NT - j * 512)
+        lds16(reinterpret_cast<const float4*>(a.pool + (size_t)tab[b][key] * HD) + x, j);
+    }
+    if (vmine)
+#pragma unroll
+      for (uint32_t j = 0; j < 2; j++) lds16(vpool + (size_t)tab[b][2 * kp + j] * (HD / 4) + dq, NK + j);
+  };
+  auto store = [&](uint8_t* buf) {
+#pragma unroll
+    for (int j = 0; j < NK; j++) {
+      const uint32_t it = j * 512 + tid, key = it / (8 * NT), x = it % (8 * NT);
+      if ((j + 1) * 512 <= 256 * NT || 64 * wave < 256 * NT - j * 512) {
+        const float4 kv = raw[512 * j + tid];
+        const float v[4] = {kv.x, kv.y, kv.z, kv.w};
+        uint32_t w[3][2];
+        split_planes<4>(v, w);
+        uint8_t* dst = buf + key * HD * 2 + (((x / 2) ^ (key % KX)) * 16 + 8 * (x % 2));
+#pragma unroll
+        for (int p = 0; p < 3; p++) *reinterpret_cast<u32x2*>(dst + p * KPL) = u32x2{w[p][0], w[p][1]};
+      }
+    }
+    if (vmine) {
+      const float4 v0 = raw[512 * NK + tid], v1 = raw[512 * (NK + 1) + tid];
+      const float v[4][2] = {{v0.x, v1.x}, {v0.y, v1.y}, {v0.z, v1.z}, {v0.w, v1.w}};
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        uint32_t w[3][1];
+        split_planes<2>(v[d], w);
+#pragma unroll
+        for (int p = 0; p < 3; p++) *reinterpret_cast<uint32_t*>(buf + vwo + d * VP + p * VPL) = w[p][0];
+      }
+    }
+  };
+  float4 qx[2 * KS];
+  {
+    const float4* qs = reinterpret_cast<const float4*>(a.qr + ((size_t)i * a.n_heads + head) * HD);
+#pragma unroll
+    for (uint32_t s = 0; s < KS; s++) {
+      qx[2 * s] = qs[4 * s + 2 * hf];
+      qx[2 * s + 1] = qs[4 * s + 2 * hf + 1];
+    }
+  }
+  __syncthreads();
+  load(0);
+  bf16x8 q[KS][3];
+#pragma unroll
+  for (uint32_t s = 0; s < KS; s++) {
+    const float4 x = qx[2 * s], y = qx[2 * s + 1];
+    const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+    uint32_t w[3][4];
+    split_planes<8>(v, w);
+#pragma unroll
+    for (int p = 0; p < 3; p++) q[s][p] = frag4(w[p]);
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  store(lds);
+  __syncthreads();
+
+  uint32_t tb = 0;
+  for (uint32_t kb = k0; kb < k1; kb += KT, tb ^= 1) {
+    const bool more = kb + KT < k1;
+    uint32_t page = 0, off = 0;
+    if (more) {
+      if (tid < KT) look(kb + 2 * KT + tid, page, off);
+      load(tb ^ 1);
+    }
+    const uint8_t* buf = lds + tb * BUF;
+    if (32 * wave < nr) {
+      f32x16 s = zero, sr = zero;  // the products of the first planes, and of the others
+#pragma unroll
+      for (uint32_t st = 0; st < KS; st++) {
+        bf16x8 kf[3];
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+          kf[p] = *reinterpret_cast<const bf16x8*>(buf + l32 * HD * 2 + p * KPL + ((2 * st + hf) ^ (l32 % KX)) * 16);
+        sr = mfma_rest(kf, q[st], sr);
+        s = mfma_bf(kf[0], q[st][0], s);
+      }
+      float mt = -INFINITY;
+#pragma unroll
+      for (uint32_t r = 0; r < 16; r++) {
+        s[r] = (s[r] + sr[r]) * sc2;
+        odd |= __builtin_amdgcn_classf(s[r], 0x207);  // NaN or infinite
+      }
+      if (kb + KT > min(pos0 + 1, k1) || kb < start1) {  // keys that some row does not attend to
+        const uint32_t p0 = kb + 4 * hf, hi = min(pos + 1, k1);
+#pragma unroll
+        for (uint32_t r = 0; r < 16; r++) {
+          const uint32_t p = p0 + 8 * (r / 4) + r % 4;
+          s[r] = p >= hi || p < start ? -INFINITY : s[r];
+        }
+      }
+#pragma unroll
+      for (uint32_t r = 0; r < 16; r++) mt = fmaxf(mt, s[r]);
+      mt = fmaxf(M, fmaxf(mt, other_half(mt)));
+      const float mu = mt == -INFINITY ? 0.0f : mt;
+      const float f = __builtin_amdgcn_exp2f(M - mu);
+      M = mt;
+      float pv[16], ps = 0.0f;
+#pragma unroll
+      for (uint32_t r = 0; r < 16; r++) {
+        pv[r] = __builtin_amdgcn_exp2f(s[r] - mu);
+        ps += pv[r];
+      }
+      L = fmaf(L, f, ps);
+      uint32_t w[2][3][4];
+      bf16x8 pf[2][3];
+#pragma unroll
+      for (int st = 0; st < 2; st++) {
+        split_planes<8>(pv + 8 * st, w[st]);
+#pragma unroll
+        for (int p = 0; p < 3; p++) pf[st][p] = frag4(w[st][p]);
+      }
+      // the tile's sum by itself, then one rounding into the row's: a long chain of them
+      // cost more than the products' own
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        f32x16 d = zero;
+        bf16x8 vf[2][3];
+#pragma unroll
+        for (int st = 0; st < 2; st++) {
+#pragma unroll
+          for (int p = 0; p < 3; p++)
+            vf[st][p] = *reinterpret_cast<const bf16x8*>(buf + 3 * KPL + (l32 + 32 * t) * VP + p * VPL + 16 * hf + 32 * st);
+          d = mfma_rest(vf[st], pf[st], d);
+        }
+        d = mfma_bf(vf[0][0], pf[0][0], d);
+        d = mfma_bf(vf[1][0], pf[1][0], d);
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[t][r] = fmaf(o[t][r], f, d[r]);
+      }
+    }
+    if (more) {
+      __builtin_amdgcn_s_waitcnt(0);  // the wave's own loads, in LDS
+      if (tid < KT) tab[tb][tid] = page * prows + off;
+      store(lds + (tb ^ 1) * BUF);
+    }
+    __syncthreads();
+  }
+  L += other_half(L);
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) odd |= __builtin_amdgcn_classf(o[t][r], 0x207);
+  odd |= other_half(odd ? 1.0f : 0.0f) != 0.0f;
+  if (mine && hf == 0) {
+    pml[2 * (size_t)prow] = odd ? __uint_as_float(kMarkSerial) : M;
+    pml[2 * (size_t)prow + 1] = L;
+  }
+  // through LDS, 32 columns at a time, so that a row's 128 bytes go out together (lane l
+  // holds 16-byte pieces of row l % 32); the wave's own 4 KB of raw, 16-byte column x of
+  // row j at x ^ (j % 8)
+  float4* w4 = raw + 256 * wave;
+  const uint32_t orow = lane / 8, ox = lane % 8;
+#pragma unroll
+  for (uint32_t t = 0; t < NT; t++) {
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++)
+      w4[8 * l32 + ((2 * j + hf) ^ (l32 % 8))] = make_float4(o[t][4 * j], o[t][4 * j + 1], o[t][4 * j + 2], o[t][4 * j + 3]);
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) {
+      const uint32_t x = 8 * j + orow;
+      const uint32_t to = __shfl(prow, x, 64);
+      if (32 * wave + x < nr) reinterpret_cast<float4*>(a.part + (size_t)to * HD)[8 * t + ox] = w4[8 * x + (ox ^ (x % 8))];
+    }
+  }
+}
+
+// Columns d .. d + 3 of query head hh of token i, position by position: for the rows that
+// k_attn_tile marks, which is rare.
+__device__ __forceinline__ float4 attn_serial(const AttnArgs& a, uint32_t i, uint32_t hh, uint32_t d) {
+  const AttnEntry e = entry(a, i);
+  const uint32_t kh = hh / (a.n_heads / a.n_kv);
+  const size_t voff = (size_t)a.bs * a.n_kv * a.hd;
+  const float* q = a.qr + ((size_t)i * a.n_heads + hh) * a.hd;
+  float M = -INFINITY, L = 0.0f, o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  bool uni = false;
+  for (uint32_t p = e.start; p <= e.pos; p++) {
+    const float* kr = key_row(a, e, p, kh);
+    float s = 0.0f;
+    for (uint32_t x = 0; x < a.hd; x++) s = fmaf(q[x], kr[x], s);
+    s *= a.scale;
+    uni |= s != s || s == INFINITY;
+    if (uni || s == -INFINITY) continue;
+    if (s > M) {
+      const float f = gm_expf(M - s);
+      L *= f;
+      for (int b = 0; b < 4; b++) o[b] *= f;
+      M = s;
+    }
+    const float pv = gm_expf(s - M);
+    L += pv;
+    for (int b = 0; b < 4; b++) o[b] = fmaf(pv, kr[voff + d + b], o[b]);
+  }
+  if (uni || M == -INFINITY)
+    return make_float4(attn_uniform(a, i, hh, d), attn_uniform(a, i, hh, d + 1), attn_uniform(a, i, hh, d + 2),
+                       attn_uniform(a, i, hh, d + 3));
+  return make_float4(o[0] / L, o[1] / L, o[2] / L, o[3] / L);
+}
+
+// The splits of a tiled call merged: a thread per four columns of a (token, head) row.
+// A marked row, or one without any score above -inf, is summed by itself.
+__global__ void __launch_bounds__(256) k_attn_merge(AttnArgs a) {
+  const uint32_t rows = a.n * a.n_heads, q4 = a.hd / 4, g = blockIdx.x * 256 + threadIdx.x, row = g / q4, x = g % q4;
+  if (row >= rows) return;
+  const float2* ml = reinterpret_cast<const float2*>(a.part + (size_t)a.nchunk * rows * a.hd) + row;
+  const float4* po = reinterpret_cast<const float4*>(a.part) + (size_t)row * q4 + x;
+  float M = -INFINITY, L = 0.0f;  // M in units of log2
+  bool serial = false;
+  for (uint32_t c = 0; c < a.nchunk; c++) {
+    const float m = ml[(size_t)c * rows].x;
+    serial |= m != m;
+    M = fmaxf(M, m);
+  }
+  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 4
+  for (uint32_t c = 0; c < a.nchunk; c++) {
+    const float2 v = ml[(size_t)c * rows];
+    if (!(v.x > -INFINITY)) continue;  // nothing was written for an empty split
+    const float f = __builtin_amdgcn_exp2f(v.x - M);
+    const float4 p = po[(size_t)c * rows * q4];
+    L = fmaf(v.y, f, L);
+    o.x = fmaf(p.x, f, o.x);
+    o.y = fmaf(p.y, f, o.y);
+    o.z = fmaf(p.z, f, o.z);
+    o.w = fmaf(p.w, f, o.w);
+  }
+  float4 w = make_float4(o.x / L, o.y / L, o.z / L, o.w / L);
+  if (serial || M == -INFINITY) w = attn_serial(a, row / a.n_heads, row % a.n_heads, 4 * x);
+  reinterpret_cast<float4*>(a.ctx)[(size_t)row * q4 + x] = w;
+}
+
 hipError_t launch_attention(const AttnArgs& a, hipStream_t st) {
   const uint32_t pairs = (a.n_heads + a.n_kv) * a.hd / 2;
   hipLaunchKernelGGL(k_rope_append, dim3(a.n, (pairs + 255) / 256), dim3(256), 0, st, a);
@@ -369,6 +795,20 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t st) {
   if (a.hd <= 128) hipLaunchKernelGGL(k_attn_partial<128>, grid, dim3(256), lds, st, a);
   else hipLaunchKernelGGL(k_attn_partial<kAttnMaxHd>, grid, dim3(256), lds, st, a);
   hipLaunchKernelGGL(k_attn_combine, dim3(a.n, a.n_heads), dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_attention_tiled(const AttnArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(k_rope_rows, dim3(a.n, 2), dim3(256), 0, st, a);
+  const dim3 grid(a.n_kv, a.ntile, a.nchunk);
+  switch (a.hd / 32) {
+    case 1: hipLaunchKernelGGL(k_attn_tile<1>, grid, dim3(512), 0, st, a); break;
+    case 2: hipLaunchKernelGGL(k_attn_tile<2>, grid, dim3(512), 0, st, a); break;
+    case 3: hipLaunchKernelGGL(k_attn_tile<3>, grid, dim3(512), 0, st, a); break;
+    default: hipLaunchKernelGGL(k_attn_tile<4>, grid, dim3(512), 0, st, a); break;
+  }
+  const uint64_t items = (uint64_t)a.n * a.n_heads * (a.hd / 4);
+  hipLaunchKernelGGL(k_attn_merge, dim3((uint32_t)((items + 255) / 256)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

@@ -400,6 +400,17 @@ struct AttnEntry {
   uint32_t fresh;   // 1: pos opens that page; the append records it in the table
 };
 
+// Rows r0 .. r0 + nr - 1 of a run: consecutive entries of one sequence from entry i0 on,
+// row r being token r / G's query head r % G of a kv head's group of G.
+struct AttnTile {
+  uint32_t i0, r0, nr;
+  uint32_t start0, pos0;  // the first token's first key and position: the tile's keys are
+  uint32_t start1, pos1;  // [start0, pos1], those that every row attends to [start1, pos0]
+  uint32_t pad;
+  const uint32_t* pages;
+};
+constexpr uint32_t kAttnTileRows = 256, kAttnTileKeys = 32;
+
 constexpr uint32_t kAttnInline = 16;  // entries carried in the kernel arguments
 struct AttnArgs {
   const AttnEntry* ent;  // [n] in device memory, or null: n <= kAttnInline entries in `inl`
@@ -413,7 +424,11 @@ struct AttnArgs {
   const float* v;        // [n][kv_dim]
   float* qr;             // [n][n_heads * hd] rotated q
   float* part;           // [n][n_heads][nchunk][hd + 2]: chunk partials (o, m, l)
-  uint32_t nchunk;       // chunks of kAttnChunk positions per entry
+  uint32_t nchunk;       // chunks of kAttnChunk positions per entry (tiled: splits of skeys)
+  const AttnTile* tiles; // tiled calls (launch_attention_tiled): [ntile], and the keys of a split;
+  const AttnEntry* hent; //   their entries and tiles in pinned host memory, which the first launch
+  const AttnTile* htile; //   copies to ent and tiles (a copy of its own cost 9.5 us a call)
+  uint32_t ntile, skeys; //   part is then [nchunk][n * n_heads][hd] o, then [nchunk][n * n_heads][2] (m, l)
   float* ctx;            // [n][n_heads * hd]
   uint32_t q_stride, kv_stride;  // floats between consecutive rows of q, and of k and v
   uint32_t nsl;                  // > 1: q, k and v are each the sum of nsl K slices of a dense
@@ -422,6 +437,9 @@ struct AttnArgs {
 
 constexpr uint32_t kAttnChunk = 64, kAttnMaxGroup = 16, kAttnMaxHd = 256;
 hipError_t launch_attention(const AttnArgs& a, hipStream_t st);
+// Runs of several tokens of one sequence (prompts): attn_tiled_hd says which head widths.
+hipError_t launch_attention_tiled(const AttnArgs& a, hipStream_t st);
+constexpr bool attn_tiled_hd(uint32_t hd) { return hd % 32 == 0 && hd <= 128; }
 
 // Decode-step glue (gmoe_glue.hip): embedding rows, residual add + RMSNorm * weight,
 // greedy token. A decode step carries its tokens in the kernel arguments.

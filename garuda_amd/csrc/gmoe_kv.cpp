@@ -13,6 +13,7 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
+#include <cstring>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -46,7 +47,8 @@ gmoe_status kfail(gmoe_status s, const char* fmt, ...) {
     if (e_ != hipSuccess) return kfail(GMOE_ERR_DEVICE, "%s failed: %s", #expr, hipGetErrorString(e_)); \
   } while (0)
 
-constexpr int kPinSlots = 8;
+constexpr size_t kPinHalf = (size_t)512 << 10;  // bytes of a half at least
+constexpr size_t kPinEntry = sizeof(AttnEntry) + sizeof(AttnTile);  // a call has at most one tile per entry
 
 struct Seq {
   bool open = false;
@@ -67,10 +69,12 @@ struct gmoe_kv {
   std::vector<Seq> seqs;
   uint8_t* scratch = nullptr; // per call: entries, rotated q, chunk partials
   size_t scratch_bytes = 0;
-  AttnEntry* pin = nullptr;   // pinned staging of the entries of calls above kAttnInline tokens, a ring
-  uint32_t pin_cap = 0;       // entries per slot
-  hipEvent_t pin_ev[kPinSlots]{};
-  int pin_slot = 0;
+  // pinned staging of the entries and tiles of calls above kAttnInline tokens: two halves,
+  // each taken from its start to its end; a half's event says its calls have read it
+  uint8_t* pin = nullptr;
+  size_t pin_half = 0, pin_at = 0;
+  hipEvent_t pin_ev[2]{};
+  int pin_cur = 0;
   uint32_t fail_reserves = 0;  // test hook: reservations still to refuse (gmoe_kv_fail_reserves)
   std::mutex mu;
 
@@ -98,14 +102,28 @@ gmoe_status grow_scratch(gmoe_kv* kv, size_t bytes) {
   return GMOE_OK;
 }
 
-gmoe_status grow_pinned(gmoe_kv* kv, uint32_t n) {
-  if (n <= kv->pin_cap) return GMOE_OK;
-  for (auto& e : kv->pin_ev) KV_TRY(hipEventSynchronize(e));
-  if (kv->pin) KV_TRY(hipHostFree(kv->pin));
-  kv->pin = nullptr;
-  const uint32_t cap = std::max(n, 256u);
-  KV_TRY(hipHostMalloc((void**)&kv->pin, kPinSlots * (size_t)cap * sizeof(AttnEntry), hipHostMallocDefault));
-  kv->pin_cap = cap;
+// `bytes` of pinned memory for a call queued on st. An event is recorded, and waited for,
+// once a half rather than once a call (5 us of idle GPU each). Calls on one cache are
+// ordered on one stream, so the one that leaves a half records for all that used it.
+gmoe_status take_pinned(gmoe_kv* kv, size_t bytes, hipStream_t st, uint8_t** out) {
+  bytes = (bytes + 63) & ~(size_t)63;
+  if (bytes > kv->pin_half) {
+    KV_TRY(hipDeviceSynchronize());  // queued calls may still read the old buffer
+    if (kv->pin) KV_TRY(hipHostFree(kv->pin));
+    kv->pin = nullptr;
+    kv->pin_half = kv->pin_at = 0;
+    const size_t half = std::max(bytes, kPinHalf);
+    KV_TRY(hipHostMalloc((void**)&kv->pin, 2 * half, hipHostMallocDefault));
+    kv->pin_half = half;
+  }
+  if (kv->pin_at + bytes > kv->pin_half) {
+    KV_TRY(hipEventRecord(kv->pin_ev[kv->pin_cur], st));
+    kv->pin_cur ^= 1;
+    kv->pin_at = 0;
+    KV_TRY(hipEventSynchronize(kv->pin_ev[kv->pin_cur]));
+  }
+  *out = kv->pin + kv->pin_cur * kv->pin_half + kv->pin_at;
+  kv->pin_at += bytes;
   return GMOE_OK;
 }
 
@@ -155,7 +173,30 @@ void commit(gmoe_kv* kv, uint32_t layer, const uint32_t* seqs, uint32_t n, AttnE
   }
 }
 
-// Scratch of a call of n entries and nchunk chunks: entries, rotated q, partials.
+// A call above kAttnInline tokens whose entries come in runs (consecutive entries of one
+// sequence: a prompt's positions) is cut into tiles of kAttnTileRows (token, query head)
+// rows. Runs shorter than an eighth of a tile on average leave the MFMA rows mostly empty and
+// take the kernels of single tokens (no tiles), as do decode batches. span receives the most keys a tile reads.
+std::vector<AttnTile> tile_runs(const gmoe_kv* kv, const AttnEntry* ent, uint32_t n, uint32_t* span) {
+  const uint32_t G = kv->d.n_heads / kv->d.n_kv_heads;
+  std::vector<AttnTile> tiles;
+  *span = 1;
+  if (n <= kAttnInline || !attn_tiled_hd(kv->d.head_dim)) return tiles;
+  for (uint32_t i = 0, j; i < n; i = j) {
+    for (j = i + 1; j < n && ent[j].pages == ent[i].pages;) j++;
+    const uint32_t rows = (j - i) * G;
+    for (uint32_t r = 0; r < rows; r += kAttnTileRows) {
+      const uint32_t nr = std::min(kAttnTileRows, rows - r);
+      const AttnEntry &f = ent[i + r / G], &e = ent[i + (r + nr - 1) / G];
+      *span = std::max(*span, e.pos + 1 - f.start);
+      tiles.push_back(AttnTile{i, r, nr, f.start, f.pos, e.start, e.pos, 0, f.pages});
+    }
+  }
+  if ((uint64_t)n * G * 8 < (uint64_t)tiles.size() * kAttnTileRows) tiles.clear();
+  return tiles;
+}
+
+// Scratch of a call of n entries and nchunk chunks: entries and tiles, rotated q, partials.
 struct AttnLayout {
   size_t o_ent, o_qr, o_part, total;
 };
@@ -164,7 +205,7 @@ AttnLayout layout(const gmoe_kv* kv, uint32_t n, uint32_t nchunk) {
   const size_t qn = (size_t)n * D.n_heads * D.head_dim;
   AttnLayout l;
   l.o_ent = 0;
-  l.o_qr = (n * sizeof(AttnEntry) + 255) & ~(size_t)255;
+  l.o_qr = (n * kPinEntry + 255) & ~(size_t)255;
   l.o_part = l.o_qr + ((qn * 4 + 255) & ~(size_t)255);
   l.total = l.o_part + (size_t)n * D.n_heads * nchunk * (D.head_dim + 2) * 4;
   return l;
@@ -195,32 +236,54 @@ AttnArgs args(const gmoe_kv* kv, uint32_t n, uint32_t nchunk, const AttnLayout& 
   return a;
 }
 
+// Workgroups a tiled call is split into at least, keys permitting.
+constexpr uint32_t kAttnTileWgs = 256;
+
 // Plans the call's entries and commits them (lengths advance and pages are taken only when
-// the whole call fits), then queues the three launches.
+// the whole call fits), then queues the launches.
 gmoe_status attend(gmoe_kv* kv, uint32_t layer, const uint32_t* seqs, uint32_t n, const float* q, const float* k,
                    const float* v, float* out, hipStream_t st, uint32_t q_stride = 0, uint32_t kv_stride = 0) {
   std::vector<AttnEntry> ent(n ? n : 1);
   uint32_t maxspan;
   if (gmoe_status s = plan(kv, layer, seqs, n, ent.data(), &maxspan)) return s;
-  const uint32_t nchunk = (maxspan + kAttnChunk - 1) / kAttnChunk;
+  uint32_t span;
+  std::vector<AttnTile> tiles = tile_runs(kv, ent.data(), n, &span);
+  if ((uintptr_t)out % 16) tiles.clear();  // its rows are written 16 bytes at a time
+  uint32_t nchunk = (maxspan + kAttnChunk - 1) / kAttnChunk, skeys = 0;
+  if (!tiles.empty()) {
+    // a tile's keys split over workgroups until the call has about one workgroup a CU,
+    // each split keeping at least two key tiles
+    const uint32_t kt = (span + kAttnTileKeys - 1) / kAttnTileKeys;
+    const uint32_t wgs = (uint32_t)tiles.size() * kv->d.n_kv_heads;
+    const uint32_t ns = std::max(1u, std::min((kAttnTileWgs + wgs - 1) / wgs, kt / 2));
+    skeys = (kt + ns - 1) / ns * kAttnTileKeys;
+    nchunk = (span + skeys - 1) / skeys;
+  }
   const AttnLayout l = layout(kv, n, nchunk);
   if (gmoe_status s = grow_scratch(kv, l.total)) return s;
+  const size_t eb = n * sizeof(AttnEntry), tb = tiles.size() * sizeof(AttnTile);
+  uint8_t* pin = nullptr;
   if (n > kAttnInline)
-    if (gmoe_status s = grow_pinned(kv, n)) return s;
+    if (gmoe_status s = take_pinned(kv, eb + tb, st, &pin)) return s;
   commit(kv, layer, seqs, n, ent.data());
   AttnArgs a = args(kv, n, nchunk, l, q, k, v, out, q_stride, kv_stride);
   if (n <= kAttnInline) {  // a decode batch: the entries ride in the kernel arguments
     std::copy(ent.begin(), ent.begin() + n, a.inl);
     a.ent = nullptr;
   } else {
-    const int h = kv->pin_slot;
-    kv->pin_slot = (h + 1) % kPinSlots;
-    KV_TRY(hipEventSynchronize(kv->pin_ev[h]));  // the slot's previous copy has been read
-    AttnEntry* pin = kv->pin + (size_t)h * kv->pin_cap;
-    std::copy(ent.begin(), ent.begin() + n, pin);
-    KV_TRY(hipMemcpyAsync(kv->scratch + l.o_ent, pin, n * sizeof(AttnEntry), hipMemcpyHostToDevice, st));
-    KV_TRY(hipEventRecord(kv->pin_ev[h], st));
+    memcpy(pin, ent.data(), eb);
+    if (tb) memcpy(pin + eb, tiles.data(), tb);
     a.ent = reinterpret_cast<const AttnEntry*>(kv->scratch + l.o_ent);
+    if (tb) {
+      a.tiles = reinterpret_cast<const AttnTile*>(kv->scratch + l.o_ent + eb);
+      a.hent = reinterpret_cast<const AttnEntry*>(pin);
+      a.htile = reinterpret_cast<const AttnTile*>(pin + eb);
+      a.ntile = (uint32_t)tiles.size();
+      a.skeys = skeys;
+      KV_TRY(launch_attention_tiled(a, st));
+      return GMOE_OK;
+    }
+    KV_TRY(hipMemcpyAsync(kv->scratch + l.o_ent, pin, eb, hipMemcpyHostToDevice, st));
   }
   KV_TRY(launch_attention(a, st));
   return GMOE_OK;

@@ -164,3 +164,66 @@ def test_nan_or_infinite_score_gives_uniform_weights(dev, bad):
             want = o.attention(0, [s], q[None], k[None], v[None])
             assert np.isfinite(got).all()
             check(got, want, f"{bad} position {pos}")
+
+
+def _prompt_calls(kv, seqs, sizes, q, k, v, per=None):
+    """The sequences' prompts, laid end to end in q, k and v: in one call, or in calls of `per` tokens."""
+    ids = [s for s, n in zip(seqs, sizes) for _ in range(n)]
+    if per is None:
+        return kv.attention(0, ids, q, k, v)
+    cut = [slice(p, min(p + per, len(ids))) for p in range(0, len(ids), per)]
+    return np.concatenate([kv.attention(0, ids[c], q[c], k[c], v[c]) for c in cut])
+
+
+@pytest.mark.parametrize("nh,nkv,hd,bs,window,sizes", [
+    (4, 1, 128, 16, 0, (17,)), (4, 1, 128, 16, 0, (32,)), (4, 1, 128, 16, 0, (33, 65)),  # tile edges: 32 tokens of 4 heads
+    (8, 8, 64, 16, 0, (127, 129)), (6, 2, 96, 8, 0, (64, 43)), (16, 1, 32, 4, 0, (21, 9)),  # group 1, 3, 16
+    (32, 8, 128, 16, 0, (300, 1)), (8, 2, 32, 16, 50, (200, 40)), (8, 2, 64, 5, 1, (70,)),  # windows, odd pages
+    (4, 4, 128, 16, 0, (600,)), (7, 1, 64, 16, 129, (400,)),
+])
+def test_prompt_tiles_equal_single_tokens(dev, nh, nkv, hd, bs, window, sizes):
+    # A call of several consecutive tokens runs tiles of 128 (token, head) rows on MFMA; the
+    # same prompt in calls of at most 16 tokens runs the single-token kernels. Both are f32
+    # softmax-weighted means of the values, so they differ by the rounding of the scores
+    # (hd products each) and of the sums over the span, relative to the largest value.
+    rng = np.random.default_rng(hd + nh + len(sizes))
+    n = sum(sizes)
+    q, k, v = (rng.normal(size=(n, w)).astype(np.float32) for w in (nh * hd, nkv * hd, nkv * hd))
+    kw = dict(block_size=bs, max_positions=700, sliding_window=window, max_seqs=2)
+    say(f"tiles nh={nh} nkv={nkv} hd={hd} bs={bs} window={window} sizes={sizes}")
+    with KvCache(dev, 1, nh, nkv, hd, **kw) as A, KvCache(dev, 1, nh, nkv, hd, **kw) as B:
+        got = _prompt_calls(A, [A.open_seq() for _ in sizes], sizes, q, k, v)
+        want = _prompt_calls(B, [B.open_seq() for _ in sizes], sizes, q, k, v, per=16)
+        # a second call on the cache the first one filled, its positions odd against the tiles
+        q2, k2, v2 = (rng.normal(size=(35, w)).astype(np.float32) for w in (nh * hd, nkv * hd, nkv * hd))
+        got2 = A.attention(0, [0] * 35, q2, k2, v2)
+        want2 = _prompt_calls(B, [0], [35], q2, k2, v2, per=16)
+    u = 2.0 ** -24
+    for gq, gk, gv, x, y in ((q, k, v, got, want), (q2, np.concatenate([k, k2]), np.concatenate([v, v2]), got2, want2)):
+        qa, ka = np.abs(gq.reshape(-1, nh, hd)), np.abs(gk.reshape(-1, nkv, hd))
+        # |q.k| / sqrt(hd) <= |q| |k| / sqrt(hd), whatever the rotation; each score is hd + 2 roundings
+        s = (np.linalg.norm(qa, axis=2).max() * np.linalg.norm(ka, axis=2).max()) / np.sqrt(hd)
+        bound = 2 * (2 * (hd + 2) * s + 700 + 32) * u * np.abs(gv).max()
+        err = np.abs(x - y).max()
+        assert err <= bound, f"err {err} bound {bound}"
+        assert np.sqrt(np.mean((x - y) ** 2)) <= 1e-6 * np.sqrt(np.mean(y ** 2)) + bound / 50
+
+
+@pytest.mark.parametrize("what", ["nan value", "inf value", "nan key", "inf key", "nan query"])
+def test_prompt_tiles_with_non_finite_rows(dev, what):
+    # A later token's non-finite key or value leaves the earlier tokens of its key tile as
+    # they are; the tokens that attend to it see what the single-token kernels give them.
+    nh, nkv, hd, n, at = 4, 2, 64, 90, 41
+    rng = np.random.default_rng(7)
+    q, k, v = (rng.normal(size=(n, w)).astype(np.float32) for w in (nh * hd, nkv * hd, nkv * hd))
+    val = np.float32("nan" if "nan" in what else "inf")
+    dict(value=v, key=k, query=q)[what.split()[1]][at, 3] = val
+    say(f"tiles with a {what}")
+    with KvCache(dev, 1, nh, nkv, hd, max_positions=128, max_seqs=1) as A, \
+            KvCache(dev, 1, nh, nkv, hd, max_positions=128, max_seqs=1) as B:
+        got = _prompt_calls(A, [A.open_seq()], [n], q, k, v)
+        want = _prompt_calls(B, [B.open_seq()], [n], q, k, v, per=16)
+    assert np.isfinite(want[:at]).all() and np.isfinite(got[:at]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    assert np.allclose(got[ok], want[ok], rtol=RTOL, atol=ATOL)
