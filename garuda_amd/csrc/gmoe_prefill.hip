@@ -608,9 +608,10 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW) k_pf(PfArgs a) {
                     for (int r = 0; r < 16; r++) acc[rt][tt][r] = __builtin_fmaf(sc, P[rt][tt][r], acc[rt][tt][r]);
               }
             }
-            // short scale groups: keep the scheduler from overlapping the next group's
-            // partial sums with these (two live sets of P do not fit the registers)
-            if constexpr (T::SU16 <= 2) __builtin_amdgcn_sched_barrier(0);
+            // short scale groups: the sums pinned here, or the unrolled steps' partial sums and
+            // products stay live together and spill (160 to 388 VGPRs; none so)
+            if constexpr (T::SU16 != 0 && T::SU16 <= 2)
+              asm volatile("" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[1][0]), "+v"(acc[1][1]));
           }
         });
         if constexpr (T::SW != 0 && C == NCH - 1) {
