@@ -21,13 +21,12 @@
 // differs from the f32 reference by reordered f32 sums (~1e-6 relative).
 //
 // Work layout. The dispatch lists the call's token tiles (kPfTok = 64 tokens of one
-// expert, in slot order) in B.ptile; blockIdx.y is a token tile. A workgroup has PF<QT>::NW
-// waves (8; 4 for Q6_K), each owning 32 rows: gate/up
-// workgroups take NW * 32 rows of f (both matrices: 256 for NW = 8), down workgroups NW *
-// 64 rows of d. Each wave owns two 32-row MFMA row tiles (gate and up of its 32 rows, or
+// expert, in slot order) in B.ptile; blockIdx.y is a token tile. A workgroup has PF<QT>::NW = 4
+// waves, each owning 32 rows: gate/up workgroups take NW * 32 rows of f (both matrices:
+// 128), down workgroups NW * 64 rows of d. Each wave owns two 32-row MFMA row tiles (gate and up of its 32 rows, or
 // two 32-row halves of its 64 down rows) and both 32-token tiles: 4 accumulators of 32x32,
-// plus 4 of partial block sums. Per chunk of K (PF<QT>::KC values: 128; 64 for Q5_K and
-// Q8_0, 32 for F16) the workgroup copies the chunk's raw 16-byte pieces of its rows (the
+// plus 4 of partial block sums. Per chunk of K (PF<QT>::KC values: 64; 128 for Q6_K, 32 for
+// F16) the workgroup copies the chunk's raw 16-byte pieces of its rows (the
 // slab's tiled layout makes each piece of 64 rows one 1 KiB run) and the tokens' hi/lo
 // activations into LDS; a lane then decodes
 // its row's 8 values of each 16-value K step straight into the MFMA B operand.
@@ -67,41 +66,48 @@ __device__ __forceinline__ void static_for(F&& f) {
 // of a unit that chunk c needs (piece(c, i) is the i-th), SU16 K16 steps per scale
 // (0: the decoded values are the weights), SW the width of a min-term sub-block, NW
 // waves per workgroup. A workgroup double-buffers its chunks, 2 x (NW * NPC KiB of
-// weight pieces + 2 * kPfTok * KC * 2 bytes of activations), within the 160 KiB of LDS.
+// weight pieces + 2 * kPfTok * KC * 2 bytes of activations). Chunks of 64 values and 4 waves
+// keep that under 80 KiB, so two workgroups share a CU and one computes while the other
+// waits for its chunk's barrier; one workgroup of 8 waves with chunks of 128 had every wave
+// of a SIMD decode, multiply and wait together. Q4_K, 512 Zipf tokens of the Mixtral shape:
+// f32 math 1073 -> 970 us, packed 1360 -> 1244; 4096 x 4096 in f32 math at 250 tokens, per
+// type: Q4_K 62 -> 45 us, Q5_K 67 -> 50, Q3_K 56 -> 44, Q2_K 63 -> 50, Q8_0 73 -> 52, Q4_0
+// 68 -> 51, F16 38 -> 36. Q6_K's pieces serve 128 values at a time, so its chunks stay 128
+// (one workgroup of 4 waves a CU; 8 waves with chunks of 64 took 83 -> 95 us there).
 // Unit byte layouts are those of the packed blocks (quant/mod.rs:624-875); Q8_0/Q4_0
 // units are eight blocks repacked as 8 f16 scales then the quants.
 // ---------------------------------------------------------------------------------
 template <int QT> struct PF;
-template <> struct PF<Q4_K> {  // d dmin | scales[12] | qs[128]: sub-blocks 4c..4c+3 in pieces 1+4c..
-  static constexpr int EU = 256, KC = 128, NPC = 5, SU16 = 16, SW = 32, NW = 8;
-  static constexpr int piece(int c, int i) { return i == 0 ? 0 : 4 * c + i; }
+template <> struct PF<Q4_K> {  // d dmin | scales[12] | qs[128]: sub-blocks 2c, 2c+1 in pieces 1+2c..
+  static constexpr int EU = 256, KC = 64, NPC = 3, SU16 = 16, SW = 32, NW = 4;
+  static constexpr int piece(int c, int i) { return i == 0 ? 0 : 2 * c + i; }
 };
 template <> struct PF<Q5_K> {  // d dmin scales | qh[32] | qs[128]: sub-blocks 2c, 2c+1 in pieces 3+2c..
-  static constexpr int EU = 256, KC = 64, NPC = 5, SU16 = 16, SW = 32, NW = 8;
+  static constexpr int EU = 256, KC = 64, NPC = 5, SU16 = 16, SW = 32, NW = 4;
   static constexpr int piece(int c, int i) { return i < 3 ? i : 2 * c + i; }
 };
 template <> struct PF<Q6_K> {  // ql[128] | qh[64] | scales[16] | d
   static constexpr int EU = 256, KC = 128, NPC = 8, SU16 = 1, SW = 0, NW = 4;
   static constexpr int piece(int c, int i) { return i < 4 ? 4 * c + i : i < 6 ? 8 + 2 * c + (i - 4) : 12 + (i - 6); }
 };
-template <> struct PF<Q3_K> {  // values regrouped (q3s_word): sub-blocks 8c.. in pieces 3c..3c+2 | scales[12] d
-  static constexpr int EU = 256, KC = 128, NPC = 4, SU16 = 16, SW = 0, NW = 8;
-  static constexpr int piece(int c, int i) { return i < 3 ? 3 * c + i : 6; }
+template <> struct PF<Q3_K> {  // values regrouped (q3s_word): sub-blocks 4c.. in two pieces of a half's three | scales[12] d
+  static constexpr int EU = 256, KC = 64, NPC = 3, SU16 = 16, SW = 0, NW = 4;
+  static constexpr int piece(int c, int i) { return i < 2 ? 3 * (c / 2) + c % 2 + i : 6; }
 };
 template <> struct PF<Q2_K> {  // scales[16] | qs[64] | d dmin
-  static constexpr int EU = 256, KC = 128, NPC = 4, SU16 = 16, SW = 16, NW = 8;
-  static constexpr int piece(int c, int i) { return i == 0 ? 0 : i < 3 ? 1 + 2 * c + (i - 1) : 5; }
+  static constexpr int EU = 256, KC = 64, NPC = 4, SU16 = 16, SW = 16, NW = 4;
+  static constexpr int piece(int c, int i) { return i == 0 ? 0 : i < 3 ? 1 + 2 * (c / 2) + (i - 1) : 5; }
 };
 template <> struct PF<Q8_0> {  // 8 scales | 8 x 32 quants: blocks 2c, 2c+1 in pieces 1+4c..4+4c
-  static constexpr int EU = 256, KC = 64, NPC = 5, SU16 = 2, SW = 0, NW = 8;
+  static constexpr int EU = 256, KC = 64, NPC = 5, SU16 = 2, SW = 0, NW = 4;
   static constexpr int piece(int c, int i) { return i == 0 ? 0 : 4 * c + i; }
 };
 template <> struct PF<Q4_0> {  // 8 scales | 8 x 16 quant bytes
-  static constexpr int EU = 256, KC = 128, NPC = 5, SU16 = 2, SW = 0, NW = 8;
-  static constexpr int piece(int c, int i) { return i == 0 ? 0 : 4 * c + i; }
+  static constexpr int EU = 256, KC = 64, NPC = 3, SU16 = 2, SW = 0, NW = 4;
+  static constexpr int piece(int c, int i) { return i == 0 ? 0 : 2 * c + i; }
 };
 template <> struct PF<F16> {  // 64 halves: values 32c.. in pieces 4c..4c+3
-  static constexpr int EU = 64, KC = 32, NPC = 4, SU16 = 0, SW = 0, NW = 8;
+  static constexpr int EU = 64, KC = 32, NPC = 4, SU16 = 0, SW = 0, NW = 4;
   static constexpr int piece(int c, int i) { return 4 * c + i; }
 };
 
@@ -282,13 +288,13 @@ template <> struct Dec<Q6_K> {
 
 // Q3_K step S (sub-block S) of chunk C: lane half h's words O(S, 2h), O(S, 2h + 1) of the
 // regrouped values v = q2 + 4 * hbit (q3s_word: the half's three words of the sub-group
-// sit at bytes 48C + 16 (x / 2) + 4 (x % 2) + 8h of the unit).
+// sit at bytes 48 (S / 8) + 16 (x / 2) + 4 (x % 2) + 8h of the unit).
 template <int C, int S>
 __device__ __forceinline__ u32x2 q3s_step(const uint8_t* row, uint32_t h) {
   constexpr int x0 = 3 * ((S % 8) / 4), k = S % 4;
   auto word = [&](auto xc) {
     constexpr int x = decltype(xc)::value;
-    return *reinterpret_cast<const uint32_t*>(pf_at<Q3_K, C, 48 * C + 16 * (x / 2) + 4 * (x % 2)>(row) + 8 * h);
+    return *reinterpret_cast<const uint32_t*>(pf_at<Q3_K, C, 48 * (S / 8) + 16 * (x / 2) + 4 * (x % 2)>(row) + 8 * h);
   };
   uint32_t b0, b1;
   if constexpr (k == 3) {
@@ -451,7 +457,7 @@ __device__ __forceinline__ void pf_block(uint32_t& bx, uint32_t& by) {
 }
 
 template <int QT, bool GU>
-__global__ void __launch_bounds__(64 * PF<QT>::NW) k_pf(PfArgs a) {
+__global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pf(PfArgs a) {
   using T = PF<QT>;
   using D = Dec<QT>;
   constexpr int NW = T::NW, NT = 64 * NW;
@@ -867,7 +873,7 @@ struct PqArgs {
 };
 
 template <int QT>
-__global__ void __launch_bounds__(64 * PF<QT>::NW) k_pq(PqArgs a) {
+__global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pq(PqArgs a) {
   using T = PF<QT>;
   using Q = PQ<QT>;
   constexpr int NW = T::NW, NT = 64 * NW;
