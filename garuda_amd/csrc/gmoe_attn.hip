@@ -12,8 +12,9 @@
 // layout, f32, so one kv head's rows of a page are contiguous. Each (sequence, layer) has
 // a page table of `ppseq` page ids. A call's entries
 // are tokens, each with its sequence's page table, its position and the position
-// attention starts at; entries of one sequence come in position order, so the append
-// kernel writes every entry's k and v before any attends (causal within the call).
+// attention starts at; entries of one sequence come in position order, and where a call has
+// several of one sequence the append kernel writes every entry's k and v before any attends
+// (causal within the call).
 // Calls of several tokens of a sequence (prompts) run tiles of rows on MFMA (k_attn_tile).
 #include "gmoe_device.h"
 
@@ -156,13 +157,26 @@ __device__ __forceinline__ float wave_sum(float v) { return wave64_sum(v); }
 // m, the sum l of exp(s - m) and o = sum of exp(s - m) * v go to part, o by float4
 // columns with the positions split over the spare threads (parts added in order).
 // Dynamic LDS: tile, q [G][hd], p [G][kAttnChunk], (m, l) [kAttnMaxGroup][2], o parts [256] float4.
+//
+// ROPE (calls whose entries are all of different sequences: decode steps): no
+// k_rope_append before it. While the chunk's rows are on their way, hd / 2 threads make the
+// position's angles (powf and sincosf, once a pair for every head) and the workgroup
+// rotates its q heads into LDS; the chunk that holds the new position also rotates and
+// stores that key and its value, and scores them from LDS. No other workgroup reads that
+// row, nor the page table's entry of a fresh page, which only it uses: positions before a
+// fresh page's first sit on other pages. The same operations as k_rope_append's, so the
+// same bits. A call of one chunk (ONE) writes the context itself, as k_attn_combine would.
+// Eight sequences over a window of 2048, four layers: 181.1 -> 170.8 us (the launch saved
+// and its gap, 35 us a layer here being the pages' 134 MB at 3.8 TB/s). The synthetic
+// engine's steps (one sequence, spans below 64: three launches a layer become one): 24
+// steps after a prompt of 16 in 8856 -> 8100 us.
 inline uint32_t attn_lds_bytes(uint32_t G, uint32_t hd) {
   return (kAttnChunk * hd + G * hd + G * kAttnChunk + 2 * kAttnMaxGroup) * 4 + 256 * 16;
 }
 
 static_assert(kAttnChunk * 4 == 256, "four threads per position of a chunk");
 
-template <int MAXHD>
+template <int MAXHD, bool ROPE, bool ONE>
 __global__ void __launch_bounds__(256) k_attn_partial(AttnArgs a) {
   constexpr int NR = MAXHD / 16;  // float4 columns of a row per thread
   extern __shared__ float4 lds_v4[];
@@ -190,25 +204,77 @@ __global__ void __launch_bounds__(256) k_attn_partial(AttnArgs a) {
   const uint32_t cnt = min(kAttnChunk, end - p0);
   const uint32_t j = t >> 2, qq = t & 3;
   const bool rowok = j < cnt;
+  const bool last = ROPE && p0 + cnt == end, rownew = last && j == cnt - 1;  // the new position's chunk and row
+  const bool rowold = rowok && !rownew;
   float4 kreg[NR], vreg[NR];
   {
-    const float* kr = key_row(a, e, p0 + (rowok ? j : 0u), h);
+    const float* kr = rowold ? key_row(a, e, p0 + j, h) : a.pool;
 #pragma unroll
     for (int r = 0; r < NR; r++) {
       const uint32_t col = qq + 4 * r;
       kreg[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       vreg[r] = kreg[r];
-      if (rowok && col < q4) {
+      if (rowold && col < q4) {
         kreg[r] = *reinterpret_cast<const float4*>(kr + 4 * col);
         vreg[r] = *reinterpret_cast<const float4*>(kr + (size_t)a.bs * kvd + 4 * col);
       }
     }
   }
-  {
+  if constexpr (ROPE) {
+    const uint32_t half = hd / 2, npair = G * half;
+    float2* ang = reinterpret_cast<float2*>(og);  // [half] (cos, sin), then the new key and value: 3 hd floats of og
+    float2 *kn = ang + half, *vn = kn + half;
+    const float* qsrc = a.q + (size_t)i * a.q_stride + (size_t)h * G * hd;
+    float x = 0.0f, y = 0.0f, nx = 0.0f, ny = 0.0f;
+    if (t < npair) ld_pair(qsrc + (t / half) * hd, t % half, a.nsl, a.sl_stride, x, y);
+    if (last && t < hd) {
+      const float* src = (t < half ? a.k : a.v) + (size_t)i * a.kv_stride + h * hd;
+      ld_pair(src, t % half, a.nsl, a.sl_stride, nx, ny);
+    }
+    if (t < half) {
+      const float freq = 1.0f / powf(a.theta, (2.0f * (float)t) / (float)hd);
+      float sn, cs;
+      sincosf((float)e.pos * freq, &sn, &cs);
+      ang[t] = make_float2(cs, sn);
+    }
+    __syncthreads();
+    for (uint32_t pr = t; pr < npair; pr += 256) {
+      if (pr != t) ld_pair(qsrc + (pr / half) * hd, pr % half, a.nsl, a.sl_stride, x, y);
+      const float2 cs = ang[pr % half];
+      reinterpret_cast<float2*>(qs)[pr] = make_float2(x * cs.x - y * cs.y, x * cs.y + y * cs.x);
+    }
+    if (last && t < hd) {
+      float* kp = a.pool + (size_t)e.page * a.page_floats + ((size_t)h * a.bs + e.pos % a.bs) * hd;
+      if (e.fresh && h == 0 && t == 0) e.pages[e.pos / a.bs] = e.page;  // for the calls after this one
+      float2 w = make_float2(nx, ny);
+      if (t < half) {
+        const float2 cs = ang[t];
+        w = make_float2(nx * cs.x - ny * cs.y, nx * cs.y + ny * cs.x);
+        kn[t] = w;
+      } else {
+        vn[t - half] = w;
+        kp += (size_t)a.bs * kvd;
+      }
+      kp[2 * (t % half)] = w.x;
+      kp[2 * (t % half) + 1] = w.y;
+    }
+    __syncthreads();
+    if (rownew) {
+#pragma unroll
+      for (int r = 0; r < NR; r++) {
+        const uint32_t col = qq + 4 * r;
+        if (col < q4) {
+          const float2 k0 = kn[2 * col], k1 = kn[2 * col + 1], v0 = vn[2 * col], v1 = vn[2 * col + 1];
+          kreg[r] = make_float4(k0.x, k0.y, k1.x, k1.y);
+          vreg[r] = make_float4(v0.x, v0.y, v1.x, v1.y);
+        }
+      }
+    }
+  } else {
     const float4* qsrc = reinterpret_cast<const float4*>(a.qr + (size_t)i * a.n_heads * hd + (size_t)h * G * hd);
     for (uint32_t x = t; x < G * q4; x += 256) reinterpret_cast<float4*>(qs)[x] = qsrc[x];
+    __syncthreads();
   }
-  __syncthreads();
   // scores of position j, every head of the group
   float acc[kAttnMaxGroup];
 #pragma unroll
@@ -281,6 +347,23 @@ __global__ void __launch_bounds__(256) k_attn_partial(AttnArgs a) {
     return o;
   };
   auto put = [&](uint32_t item, float4 o) {
+    if constexpr (ONE) {
+      const uint32_t g = item / q4, col = 4 * (item % q4);
+      const float m = ml(g, 0), l = ml(g, 1);
+      if (m != m || m == -INFINITY) {  // attn_uniform's plain mean, from the tile
+        const float u = fdiv(1.0f, (float)cnt);
+        o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (uint32_t jj = 0; jj < cnt; jj++) {
+          const float4 v = tile4[jj * q4 + item % q4];
+          o = make_float4(o.x + v.x * u, o.y + v.y * u, o.z + v.z * u, o.w + v.w * u);
+        }
+      } else {  // 0 + o, as the combine's first chunk gives (a -0 sum becomes +0)
+        o = make_float4((0.0f + o.x) / l, (0.0f + o.y) / l, (0.0f + o.z) / l, (0.0f + o.w) / l);
+      }
+      float* dst = a.ctx + ((size_t)i * a.n_heads + h * G + g) * hd + col;
+      dst[0] = o.x; dst[1] = o.y; dst[2] = o.z; dst[3] = o.w;
+      return;
+    }
     float* dst = out + (item / q4) * gstride + 4 * (item % q4);
     dst[0] = o.x; dst[1] = o.y; dst[2] = o.z; dst[3] = o.w;
   };
@@ -302,7 +385,7 @@ __global__ void __launch_bounds__(256) k_attn_partial(AttnArgs a) {
   } else {
     for (uint32_t x = t; x < items; x += 256) put(x, pv_sum(x, 0, cnt));
   }
-  if (t < G) {
+  if (!ONE && t < G) {
     out[t * gstride + hd] = ml(t, 0);
     out[t * gstride + hd + 1] = ml(t, 1);
   }
@@ -781,19 +864,45 @@ __global__ void __launch_bounds__(256) k_attn_merge(AttnArgs a) {
   reinterpret_cast<float4*>(a.ctx)[(size_t)row * q4 + x] = w;
 }
 
-hipError_t launch_attention(const AttnArgs& a, hipStream_t st) {
-  const uint32_t pairs = (a.n_heads + a.n_kv) * a.hd / 2;
-  hipLaunchKernelGGL(k_rope_append, dim3(a.n, (pairs + 255) / 256), dim3(256), 0, st, a);
+template <bool ROPE, bool ONE>
+static void launch_partial(const AttnArgs& a, hipStream_t st) {
   static const bool once =
-      hipFuncSetAttribute((const void*)k_attn_partial<128>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      hipFuncSetAttribute((const void*)k_attn_partial<128, ROPE, ONE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)attn_lds_bytes(kAttnMaxGroup, 128)) == hipSuccess &&
-      hipFuncSetAttribute((const void*)k_attn_partial<kAttnMaxHd>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      hipFuncSetAttribute((const void*)k_attn_partial<kAttnMaxHd, ROPE, ONE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)attn_lds_bytes(kAttnMaxGroup, kAttnMaxHd)) == hipSuccess;
   (void)once;
   const dim3 grid(a.n, a.n_kv, a.nchunk);
   const uint32_t lds = attn_lds_bytes(a.n_heads / a.n_kv, a.hd);
-  if (a.hd <= 128) hipLaunchKernelGGL(k_attn_partial<128>, grid, dim3(256), lds, st, a);
-  else hipLaunchKernelGGL(k_attn_partial<kAttnMaxHd>, grid, dim3(256), lds, st, a);
+  if (a.hd <= 128) hipLaunchKernelGGL((k_attn_partial<128, ROPE, ONE>), grid, dim3(256), lds, st, a);
+  else hipLaunchKernelGGL((k_attn_partial<kAttnMaxHd, ROPE, ONE>), grid, dim3(256), lds, st, a);
+}
+
+// Whether the context's floats overlap those of `rows` rows of q, k or v (all their slices).
+static bool ctx_overlaps(const AttnArgs& a, const float* p, uint32_t width, uint32_t stride) {
+  const uintptr_t c0 = (uintptr_t)a.ctx, c1 = c0 + (size_t)a.n * a.n_heads * a.hd * 4, p0 = (uintptr_t)p;
+  const uintptr_t p1 = p0 + (((size_t)a.n - 1) * stride + width + (a.nsl > 1 ? (a.nsl - 1) * a.sl_stride : 0)) * 4;
+  return c0 < p1 && p0 < c1;
+}
+
+hipError_t launch_attention(const AttnArgs& a, hipStream_t st) {
+  // The fused first launch needs every key but an entry's own in the pages already: entries
+  // of different sequences. One chunk then needs no other launch, unless the context lies
+  // over an input that a workgroup of another head or token has yet to read.
+  const uint32_t qd = a.n_heads * a.hd, kvd = a.n_kv * a.hd;
+  const bool one = a.nchunk == 1 && !ctx_overlaps(a, a.q, qd, a.q_stride) && !ctx_overlaps(a, a.k, kvd, a.kv_stride) &&
+                   !ctx_overlaps(a, a.v, kvd, a.kv_stride);
+  if (a.distinct && one) {
+    launch_partial<true, true>(a, st);
+    return hipGetLastError();
+  }
+  if (a.distinct) {
+    launch_partial<true, false>(a, st);
+  } else {
+    const uint32_t pairs = (a.n_heads + a.n_kv) * a.hd / 2;
+    hipLaunchKernelGGL(k_rope_append, dim3(a.n, (pairs + 255) / 256), dim3(256), 0, st, a);
+    launch_partial<false, false>(a, st);
+  }
   hipLaunchKernelGGL(k_attn_combine, dim3(a.n, a.n_heads), dim3(256), 0, st, a);
   return hipGetLastError();
 }

@@ -416,6 +416,7 @@ struct AttnArgs {
   const AttnEntry* ent;  // [n] in device memory, or null: n <= kAttnInline entries in `inl`
   AttnEntry inl[kAttnInline];
   uint32_t n, n_heads, n_kv, hd, bs;
+  uint32_t distinct;     // 1: no two entries are of one sequence
   float theta, scale;
   float* pool;           // page pool
   uint64_t page_floats;  // 2 * bs * kv_dim

@@ -270,6 +270,10 @@ gmoe_status attend(gmoe_kv* kv, uint32_t layer, const uint32_t* seqs, uint32_t n
   if (n <= kAttnInline) {  // a decode batch: the entries ride in the kernel arguments
     std::copy(ent.begin(), ent.begin() + n, a.inl);
     a.ent = nullptr;
+    a.distinct = 1;
+    for (uint32_t i = 0; i < n; i++)
+      for (uint32_t j = 0; j < i; j++)
+        if (ent[j].pages == ent[i].pages) a.distinct = 0;
   } else {
     memcpy(pin, ent.data(), eb);
     if (tb) memcpy(pin + eb, tiles.data(), tb);
@@ -456,6 +460,7 @@ gmoe_status kv_attend_dev(gmoe_kv* kv, uint32_t n, const AttnEntry* d_ent, uint3
   if (nsl > kMaxKsg) return kfail(GMOE_ERR_INFERENCE, "%u K slices exceed %u", nsl, kMaxKsg);
   AttnArgs a = args(kv, n, nchunk, l, q, k, v, out, q_stride, kv_stride);
   a.ent = d_ent;
+  a.distinct = 1;  // a decode step's sequences, which kv_check_step refuses twice
   a.nsl = nsl;
   a.sl_stride = sl_stride;
   KV_TRY(launch_attention(a, st));

@@ -227,3 +227,52 @@ def test_prompt_tiles_with_non_finite_rows(dev, what):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
     ok = np.isfinite(want)
     assert np.allclose(got[ok], want[ok], rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("nh,nkv,hd,bs,window,bad", [
+    (8, 2, 32, 16, 0, None), (32, 8, 128, 16, 70, None), (2, 2, 4, 8, 0, None), (16, 1, 256, 16, 0, None),
+    (8, 2, 96, 16, 64, None), (32, 8, 128, 16, 0, "nan"), (8, 2, 32, 5, 0, "inf")])
+def test_decode_launch_with_rotation_is_the_same_bits(dev, nh, nkv, hd, bs, window, bad):
+    # Calls of different sequences rotate and append in the attention's own launch; a call
+    # with a sequence twice takes the separate launches. Both run the same operations, so
+    # rows of sequences 0 and 1 agree bit for bit across pages and chunks of 64 positions.
+    rng = np.random.default_rng(hd + bs)
+    with KvCache(dev, 1, nh, nkv, hd, block_size=bs, max_positions=400, sliding_window=window, max_seqs=3) as A, \
+            KvCache(dev, 1, nh, nkv, hd, block_size=bs, max_positions=400, sliding_window=window, max_seqs=3) as B:
+        a = [A.open_seq() for _ in range(2)]
+        b = [B.open_seq() for _ in range(3)]
+        for step in range(134):
+            q, k, v = (rng.normal(size=(4, w)).astype(np.float32) for w in (nh * hd, nkv * hd, nkv * hd))
+            if bad and step in (20, 90):
+                q[0, 3], k[1, 2] = np.float32(bad), -np.float32(bad)
+            n = 1 if step == 0 else 2  # the second sequence runs one position behind
+            got = A.attention(0, a[:n], q[:n], k[:n], v[:n])
+            want = B.attention(0, b[:n] + [b[2]] * 2, *(np.concatenate([x[:n], x[2:]]) for x in (q, k, v)))[:n]
+            if step % 16 == 0 or 60 <= step < 68 or step > 126:
+                say(f"step {step}")
+            same = (bits(got) == bits(want)) | (np.isnan(got) & np.isnan(want))
+            assert same.all(), f"step {step}: {np.count_nonzero(~same)} differ"
+
+
+def test_decode_context_over_its_query(dev):
+    # the context may lie over the call's q, as when a caller reuses the buffer
+    import ctypes as C
+    hip = _hip()
+    nh, nkv, hd, n = 8, 2, 64, 3
+    rng = np.random.default_rng(5)
+    qkv = [rng.normal(size=(n, w)).astype(np.float32) for w in (nh * hd, nkv * hd, nkv * hd)]
+    with KvCache(dev, 1, nh, nkv, hd) as A, KvCache(dev, 1, nh, nkv, hd) as B:
+        want = A.attention(0, [A.open_seq() for _ in range(n)], *qkv)
+        bufs = [C.c_void_p() for _ in range(3)]
+        for buf, x in zip(bufs, qkv):
+            assert hip.hipMalloc(C.byref(buf), x.nbytes) == 0
+            assert hip.hipMemcpy(buf, x.ctypes.data, x.nbytes, 1) == 0
+        try:
+            B.attention_async(0, [B.open_seq() for _ in range(n)], *(x.value for x in bufs), bufs[0].value, 0)
+            assert hip.hipDeviceSynchronize() == 0
+            got = np.empty_like(want)
+            assert hip.hipMemcpy(got.ctypes.data, bufs[0], got.nbytes, 2) == 0
+            assert np.array_equal(bits(got), bits(want))
+        finally:
+            for buf in bufs:
+                hip.hipFree(buf)
