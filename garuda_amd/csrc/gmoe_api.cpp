@@ -756,8 +756,8 @@ gmoe_status check_ctx(gmoe_ctx* c) {
 // ---- dense projections: Weight::matmul_rows(0, xs, n, out) (llama/mod.rs:160-195) ----
 // The weight is the one "expert" of a down product: decode-sized calls quantise the
 // activations per 32 (packed math) or read them as f32 and run the K-split down kernel;
-// prefill-sized f32-math calls run it on MFMA over token tiles; the K slices are then
-// added in order into out [n][rows].
+// prefill-sized calls run it on MFMA over token tiles (f32 math: k_pf; packed: k_pq); the
+// K slices are then added in order into out [n][rows].
 LayerDev dense_dev(const Dense& W) {
   LayerDev D{};
   D.d = W.rows;
@@ -772,7 +772,7 @@ LayerDev dense_dev(const Dense& W) {
 struct DenseCarve {
   FwdBufs B;
   uint32_t ksg;
-  bool pf, int8;
+  bool pf, pq, int8;
 };
 
 constexpr uint32_t kDenseFuseKsg = 4;
@@ -781,11 +781,13 @@ constexpr uint32_t kDenseFuseKsg = 4;
 size_t plan_dense(const gmoe_ctx* c, const Dense& W, uint32_t n, uint8_t* base, DenseCarve* out) {
   const LayerDev D = dense_dev(W);
   const bool pf = prefill_dense_ok(D, n);
-  const bool int8 = !pf && uses_int8(W.math, W.qtype);
+  const bool pq = !pf && pq_dense_ok(D, n);
+  const bool int8 = !pf && !pq && uses_int8(W.math, W.qtype);
   FwdBufs B{};
   B.nslot = n;
-  B.ptile_cap = pf ? (n + kPfTok - 1) / kPfTok : 0;
-  const uint32_t ksg = pf ? 0u : dense_ksg(D);  // prefill: from the carved buffers below
+  B.ptile_cap = pf || pq ? (n + kPfTok - 1) / kPfTok : 0;
+  B.nkp = n + kPfTok;  // a token tile's kPfTok factors are always in bounds
+  const uint32_t ksg = pf || pq ? 0u : dense_ksg(D);  // MFMA: from the carved buffers below
   ScratchPlan P;
   const size_t nx = (size_t)n * W.cols;
   size_t o_work = P.add(sizeof(ExpertWork)), o_off = P.add(8), o_act = P.add(8), o_tok = P.add((size_t)n * 4),
@@ -804,13 +806,19 @@ size_t plan_dense(const gmoe_ctx* c, const Dense& W, uint32_t n, uint8_t* base, 
     o_xh = P.add(2 * nx * 2);
     o_xsh = P.add(2 * (nx / 16) * 2);
   }
+  size_t o_qxs = 0, o_qxsum = 0;
+  if (pq) {
+    o_xh = P.add(nx * 2);
+    o_qxs = P.add((size_t)(W.cols / 32) * B.nkp * 4);
+    o_qxsum = P.add((size_t)(W.cols / 16) * B.nkp * 4);
+  }
   const size_t o_y = P.add((size_t)kMaxKsg * n * W.rows * 4);
   if (base && out) {
     B.work = (ExpertWork*)(base + o_work);
     B.offsets = (uint32_t*)(base + o_off);
     B.active = (uint32_t*)(base + o_act);
     B.slot_tok = (uint32_t*)(base + o_tok);
-    B.ptile = pf ? (uint32_t*)(base + o_pt) : nullptr;
+    B.ptile = pf || pq ? (uint32_t*)(base + o_pt) : nullptr;
     if (int8 && !fuse) {
       B.hq = (int8_t*)(base + o_q);
       B.hsc = (float*)(base + o_s);
@@ -820,16 +828,22 @@ size_t plan_dense(const gmoe_ctx* c, const Dense& W, uint32_t n, uint8_t* base, 
       B.xh = B.hh = (_Float16*)(base + o_xh);
       B.xsh = B.hsh = (_Float16*)(base + o_xsh);
     }
+    if (pq) {
+      B.xh = (_Float16*)(base + o_xh);
+      B.qxs = (float*)(base + o_qxs);
+      B.qxsum = (float*)(base + o_qxsum);
+    }
     B.y = (float*)(base + o_y);
     if (n <= kDenseTab) {  // the precomputed tables: no setup launch
       B.work = W.work_tab + (n - 1);
       B.slot_tok = c->ident;
-      if (pf) B.ptile = c->ident;
+      if (pf || pq) B.ptile = c->ident;
     }
     out->B = B;
     out->pf = pf;
+    out->pq = pq;
     out->int8 = int8;
-    out->ksg = pf ? prefill_ksg(D, B) : ksg;
+    out->ksg = pf ? prefill_ksg(D, B) : pq ? pq_dense_ksg(D, B) : ksg;
   }
   return P.total;
 }
@@ -846,6 +860,9 @@ gmoe_status run_dense(const Dense& W, const DenseCarve& cv, const float* x, uint
     B.hs = x;
     HIP_TRY(launch_gather_f16(Gd, B, n, st));
     HIP_TRY(launch_prefill_down(D, B, n, cv.ksg, st));
+  } else if (cv.pq) {
+    HIP_TRY(launch_quant_codes(D, B, x, n, st));
+    HIP_TRY(launch_pq_dense(D, B, n, cv.ksg, st));
   } else {
     if (cv.int8 && B.hq) {
       HIP_TRY(launch_quant_act(x, n, W.cols, B.hq, B.hsc, B.hsum, W.qtype, st));

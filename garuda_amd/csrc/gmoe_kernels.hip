@@ -1544,6 +1544,48 @@ __global__ void __launch_bounds__(256) k_gather_codes(const int8_t* __restrict__
   }
 }
 
+// The same from f32 rows (a dense call's tokens in order): each thread quantises its block
+// with quant32's arithmetic first, so no codes go to memory between.
+__global__ void __launch_bounds__(256) k_quant_codes(const float* __restrict__ x, uint32_t d, uint32_t nk, uint32_t nkp,
+                                                     uint32_t sw, _Float16* __restrict__ xh, float* __restrict__ qxs,
+                                                     float* __restrict__ qxsum) {
+  typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+  const uint32_t s = blockIdx.x * 64 + (threadIdx.x & 63), b = blockIdx.y * 4 + (threadIdx.x >> 6), nb = d / 32;
+  if (s >= nk || b >= nb) return;
+  const float4* p = reinterpret_cast<const float4*>(x + (size_t)s * d + 32 * b);
+  float v[32];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const float4 t = p[i];
+    v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+  }
+  uint32_t packed[8];
+  float scale;
+  int sum0, sum1;
+  quant32_regs(v, packed, &scale, &sum0, &sum1);
+  half8* dst = reinterpret_cast<half8*>(xh + (size_t)s * d + 32 * b);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    half8 o;
+#pragma unroll
+    for (int j = 0; j < 8; j++) o[j] = (_Float16)(float)(int8_t)(packed[2 * i + j / 4] >> (8 * (j % 4)));
+    dst[i] = o;
+  }
+  qxs[(size_t)b * nkp + s] = scale;
+  if (sw == 32) {
+    qxsum[(size_t)b * nkp + s] = (float)(sum0 + sum1);
+  } else if (sw == 16) {
+    qxsum[(size_t)(2 * b) * nkp + s] = (float)sum0;
+    qxsum[(size_t)(2 * b + 1) * nkp + s] = (float)sum1;
+  }
+}
+
+hipError_t launch_quant_codes(const LayerDev& L, const FwdBufs& B, const float* x, uint32_t n, hipStream_t st) {
+  hipLaunchKernelGGL(k_quant_codes, dim3((n + 63) / 64, (L.f / 32 + 3) / 4), dim3(256), 0, st, x, L.f, n, B.nkp,
+                     pq_sum_width(L.qt_down), B.xh, B.qxs, B.qxsum);
+  return hipGetLastError();
+}
+
 hipError_t launch_gather_codes(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st) {
   const uint32_t nk = n * L.k;
   hipLaunchKernelGGL(k_gather_codes, dim3((nk + 63) / 64, (L.d / 32 + 3) / 4), dim3(256), 0, st, B.xq, B.xs, B.xsum,
@@ -1556,6 +1598,35 @@ hipError_t launch_pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hip
 #define GU(T) case T: return pq_gateup<T>(L, B, n, st);
     GU(Q4_K) GU(Q5_K) GU(Q6_K) GU(Q3_K) GU(Q2_K) GU(Q8_0)
 #undef GU
+  }
+  return hipErrorInvalidValue;
+}
+
+// Tokens from which a packed-math dense call runs on MFMA. The decode kernels' time grows
+// with every 8 tokens, a token tile's hardly: two layers' q|k|v and o (Q4_K, 6144 and 4096
+// rows of 4096) take 83.7 us there and about 85 here at 16 tokens, 110 and 88.6 at 24, 227
+// and 131 at 64, 791 and 193 at 256; the head (Q6_K, 32000 rows) 132 and 96 at 24, 313 and
+// 166 at 64.
+constexpr uint32_t kPqDenseMin = 24;
+
+bool pq_dense_ok(const LayerDev& L, uint32_t n) {
+  return L.math == 0 && n >= kPqDenseMin && pq_type_rt(L.qt_down) && L.d % 256 == 0 && L.f % 256 == 0;
+}
+
+uint32_t pq_dense_ksg(const LayerDev& L, const FwdBufs& B) {
+  switch (L.qt_down) {
+#define DN(T) case T: return pq_dense_slices<T>(L, B);
+    DN(Q4_K) DN(Q5_K) DN(Q6_K) DN(Q3_K) DN(Q2_K) DN(Q8_0)
+#undef DN
+  }
+  return 1;
+}
+
+hipError_t launch_pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, hipStream_t st) {
+  switch (L.qt_down) {
+#define DN(T) case T: return pq_dense<T>(L, B, n, ksg, st);
+    DN(Q4_K) DN(Q5_K) DN(Q6_K) DN(Q3_K) DN(Q2_K) DN(Q8_0)
+#undef DN
   }
   return hipErrorInvalidValue;
 }

@@ -712,7 +712,8 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pf(PfArgs a) {
 // Inputs: the activation codes in slot order as fp16 ([nk][K]), and the per-token
 // factors transposed, [K/32][nkp] scales and [K/SW][nkp] sums (nkp >= nk + 64 so a
 // token tile's 64 slots are always in bounds). Gate/up writes h's codes, scales and
-// sums the same way for the down product.
+// sums the same way for the down product. A dense projection (k_pq<QT, false>) keeps the
+// terms in K order within a slice of K.
 // ---------------------------------------------------------------------------------
 template <int QT> struct PQ;
 
@@ -864,6 +865,8 @@ struct PqArgs {
   const float* ins;     // [K/32][nkp] activation scales
   const float* insum;   // [K/SWS][nkp] activation sums (types with SWS)
   uint32_t nk, nkp, K, rows;
+  uint32_t upk;         // dense: units of K per slice
+  float* y;             // dense: [slices][nk][rows]
   // h dequantised (scale * q of its int8 requantisation) as fp16 hi/lo planes [2][nk][rows],
   // and its sums over swf rows as hi/lo planes [2][nk][rows/swf] (swf 0: none): the input
   // of the f32-math down product (k_pf)
@@ -872,7 +875,10 @@ struct PqArgs {
   uint32_t swf;
 };
 
-template <int QT>
+// GU: gate/up, the whole of K in one workgroup. !GU: a dense projection (rows of one
+// matrix, units [u0, u1) of K per blockIdx.z slice, output y slice blockIdx.z), tiled as
+// k_pf's down product.
+template <int QT, bool GU>
 __global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pq(PqArgs a) {
   using T = PF<QT>;
   using Q = PQ<QT>;
@@ -889,8 +895,8 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pq(PqArgs a) {
   static_assert(2 * BUF <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(16))) uint8_t lds[2 * BUF];
 
-  uint32_t bx, by;
-  pf_block(bx, by);
+  uint32_t bx = blockIdx.x, by = blockIdx.y;
+  if constexpr (GU) pf_block(bx, by);
   const uint32_t pt = a.ptile[by];
   if (pt == ~0u) return;
   const ExpertWork* W = a.work + (pt >> 16);
@@ -899,17 +905,17 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pq(PqArgs a) {
   const uint32_t tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t K = a.K, nunit = K / T::EU;
-  const uint32_t u0 = 0, u1 = nunit;
+  const uint32_t u0 = GU ? 0 : blockIdx.z * a.upk, u1 = GU ? nunit : min(nunit, u0 + a.upk);
 
-  // NW/2 gate tiles then NW/2 up tiles of 64 rows; wave w owns rows 32 (w % 2) .. of gate
-  // tile w / 2 (rt = 0) and of the same up tile (rt = 1)
+  // GU: NW/2 gate tiles then NW/2 up tiles of 64 rows; wave w owns rows 32 (w % 2) .. of gate
+  // tile w / 2 (rt = 0) and of the same up tile (rt = 1). !GU: NW tiles, wave w owns tile w
   const size_t tile_bytes = (size_t)nunit * kTileRows * U;
-  const uint8_t* m_lo = W->w[0] + (NW / 2) * bx * tile_bytes;
-  const uint8_t* m_hi = W->w[1] + (NW / 2) * bx * tile_bytes;
+  const uint8_t* m_lo = GU ? W->w[0] + (NW / 2) * bx * tile_bytes : W->w[2] + NW * bx * tile_bytes;
+  const uint8_t* m_hi = GU ? W->w[1] + (NW / 2) * bx * tile_bytes : m_lo + (NW / 2) * tile_bytes;
   uint32_t row[2];
 #pragma unroll
   for (int rt = 0; rt < 2; rt++) {
-    const uint32_t tm = rt * (NW / 2) + wave / 2, i = 32 * (wave % 2) + l32;
+    const uint32_t tm = GU ? rt * (NW / 2) + wave / 2 : wave, i = GU ? 32 * (wave % 2) + l32 : 32 * rt + l32;
     row[rt] = (tm * NPC * 64 + i) * 16;
   }
   const uint32_t xrow = l32 * NCK * 16;
@@ -1028,7 +1034,12 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pq(PqArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       const uint32_t t = 32 * tt + 8 * (r / 4) + 4 * h + (r % 4);
-      {
+      if constexpr (!GU) {
+        float* y = a.y + (size_t)blockIdx.z * a.nk * a.rows;
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+          if (t < m) y[(size_t)(s0 + t) * a.rows + bx * 64 * NW + 64 * wave + 32 * rt + l32] = acc[rt][tt][r];
+      } else {
         // h = silu(g) * u, then quantised per 32 rows (the 32 lanes of this half) with
         // quant_wave's arithmetic (quant/mod.rs:331-345)
         const uint32_t fr = bx * WROWS + 32 * wave + l32;
@@ -1095,7 +1106,48 @@ hipError_t pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_
     a.outf = B.hh;
     a.outfs = B.hsh;
     a.swf = pf_sum_width(L.qt_down);
-    hipLaunchKernelGGL((k_pq<QT>), dim3(L.f / pf_rows<QT>(true), B.ptile_cap), dim3(64 * PF<QT>::NW), 0, st, a);
+    hipLaunchKernelGGL((k_pq<QT, true>), dim3(L.f / pf_rows<QT>(true), B.ptile_cap), dim3(64 * PF<QT>::NW), 0, st, a);
+    return hipGetLastError();
+  }
+}
+
+// K slices of the packed-math dense product: two workgroups a CU at once, as fit its LDS,
+// each slice keeping at least two units.
+template <int QT>
+uint32_t pq_dense_slices(const LayerDev& L, const FwdBufs& B) {
+  if constexpr (!pq_type<QT>()) {
+    return 1;
+  } else {
+    const uint32_t tiles = (L.d / pf_rows<QT>(false)) * B.ptile_cap, nunit = L.f / PF<QT>::EU;
+    const uint32_t ks = min(min((2 * 256 + tiles - 1) / tiles, max(1u, nunit / 2)), kMaxKsg);
+    const uint32_t upk = (nunit + ks - 1) / ks;
+    return (nunit + upk - 1) / upk;
+  }
+}
+
+// A dense projection in packed math: the reference's int8 dots and terms, in K order
+// within a slice.
+template <int QT>
+hipError_t pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, hipStream_t st) {
+  if constexpr (!pq_type<QT>()) {
+    return hipErrorNotSupported;
+  } else {
+    if (L.d % pf_rows<QT>(false) || L.f % PF<QT>::EU || ksg < 1 || ksg > kMaxKsg) return hipErrorInvalidValue;
+    PqArgs a{};
+    a.work = B.work;
+    a.ptile = B.ptile;
+    a.in = B.xh;
+    a.ins = B.qxs;
+    a.insum = B.qxsum;
+    a.nk = n;
+    a.nkp = B.nkp;
+    a.K = L.f;
+    a.rows = L.d;
+    const uint32_t nunit = L.f / PF<QT>::EU;
+    a.upk = (nunit + ksg - 1) / ksg;
+    a.y = B.y;
+    hipLaunchKernelGGL((k_pq<QT, false>), dim3(L.d / pf_rows<QT>(false), B.ptile_cap, ksg), dim3(64 * PF<QT>::NW), 0,
+                       st, a);
     return hipGetLastError();
   }
 }
@@ -1164,5 +1216,7 @@ template uint32_t prefill_down_slices<GMOE_QT>(const LayerDev&, const FwdBufs&);
 template hipError_t prefill_gateup<GMOE_QT>(const LayerDev&, const FwdBufs&, uint32_t, hipStream_t);
 template hipError_t prefill_down<GMOE_QT>(const LayerDev&, const FwdBufs&, uint32_t, uint32_t, hipStream_t);
 template hipError_t pq_gateup<GMOE_QT>(const LayerDev&, const FwdBufs&, uint32_t, hipStream_t);
+template uint32_t pq_dense_slices<GMOE_QT>(const LayerDev&, const FwdBufs&);
+template hipError_t pq_dense<GMOE_QT>(const LayerDev&, const FwdBufs&, uint32_t, uint32_t, hipStream_t);
 
 }  // namespace gmoe

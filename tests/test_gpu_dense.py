@@ -210,3 +210,13 @@ def test_dense_refusals(dev):
     W.release()
     with pytest.raises(G.InferenceError):
         W.matmul_rows(np.zeros((2, 256), np.float32))
+
+
+@pytest.mark.parametrize("qtype", [G.Q4_K, G.Q5_K, G.Q6_K, G.Q3_K, G.Q2_K, G.Q8_0])
+def test_dense_packed_on_mfma(dev, qtype):
+    # rows and columns a multiple of 256 from 24 tokens on: k_pq's dots, terms and slices, with
+    # half token tiles, ragged last ones, one unit a row and a call past the table of 2048
+    check(dev, qtype, 256, 256, (23, 24, 33, 63, 65, 130), G.MATH_PACKED, seed=5)
+    check(dev, qtype, 768, 1792, (32, 97), G.MATH_PACKED, seed=6)
+    if qtype == G.Q4_K:
+        check(dev, qtype, 256, 512, (2048, 2049), G.MATH_PACKED, seed=7)
