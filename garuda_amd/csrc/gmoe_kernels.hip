@@ -1499,13 +1499,18 @@ static bool pq_type_rt(uint32_t qt) {
   return qt == Q4_K || qt == Q5_K || qt == Q6_K || qt == Q3_K || qt == Q2_K || qt == Q8_0;
 }
 
-// Tokens per expert from which the MFMA products beat the per-row decode kernels
-// (whose cost grows with every token an expert gets, while a token tile's is fixed).
-constexpr uint32_t kPqMinPerExpert = 16;
+// Tokens per expert from which the MFMA products beat the per-row decode kernels (whose
+// cost grows with every 8 tokens an expert gets, while a token tile's hardly does). Mixtral
+// shape, decode kernels and MFMA: Q4_K 32 tokens (8 an expert) 367 and 368 us, 48 tokens 536
+// and 390, 63 tokens 687 and 400; Q3_K gate/up 32 tokens 365 and 445, 48 tokens 515 and 483, 63
+// tokens 677 and 492.
+// 128 experts of 2048 x 768 at 12 an expert: Q4_K 258 and 195, Q3_K 270 and 225; Q6_K, one
+// workgroup a CU: 329 and 405, equal at 16.
+constexpr uint32_t pq_min_per_expert(uint32_t qt) { return qt == Q4_K || qt == Q3_K ? 12 : 16; }
 
 bool prefill_packed_ok(const LayerDev& L, uint32_t n) {
   const uint32_t nk = n * L.k;
-  return L.math == 0 && nk >= kPfMinSlots && nk >= kPqMinPerExpert * L.ne && L.qt_gate == L.qt_up &&
+  return L.math == 0 && nk >= kPfMinSlots && nk >= pq_min_per_expert(L.qt_gate) * L.ne && L.qt_gate == L.qt_up &&
          pq_type_rt(L.qt_gate) && pq_type_rt(L.qt_down) && L.d % 512 == 0 && L.f % 256 == 0 && L.ne < 65536;
 }
 

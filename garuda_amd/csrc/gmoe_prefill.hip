@@ -875,16 +875,31 @@ struct PqArgs {
   uint32_t swf;
 };
 
+// Waves a SIMD of k_pq. The term's chain of VALU operations bounds it and two waves leave the
+// SIMD waiting half the time, so gate/up takes three workgroups a CU where their LDS fits
+// (Q4_K, Q3_K, Q2_K), within 168 VGPRs: one 32-token tile's dots are live at a time. Zipf
+// tokens of the Mixtral shape, packed math: Q4_K 512 tokens 1195 -> 1094 us, 120 tokens 634
+// -> 542; Q3_K gate/up 1559 -> 1456 and 823 -> 734. Where three do not fit, and in a dense
+// call, whose K slices make two workgroups a CU, both tiles' dots are made before the
+// terms: the other order cost the Q6_K head at 64 tokens 166 -> 172 us.
+template <int QT, bool GU>
+constexpr int pq_waves() {
+  constexpr int KC = PF<QT>::KC;
+  constexpr int BUF = PF<QT>::NW * PF<QT>::NPC * 1024 + (int)kPfTok * (KC * 2 + 4 * (KC / 32 + (PQ<QT>::SWS ? KC / PQ<QT>::SWS : 0)));
+  return GU && 3 * 2 * BUF <= 160 * 1024 ? 3 : 2;
+}
+
 // GU: gate/up, the whole of K in one workgroup. !GU: a dense projection (rows of one
 // matrix, units [u0, u1) of K per blockIdx.z slice, output y slice blockIdx.z), tiled as
 // k_pf's down product.
 template <int QT, bool GU>
-__global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pq(PqArgs a) {
+__global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU>())) k_pq(PqArgs a) {
   using T = PF<QT>;
   using Q = PQ<QT>;
   constexpr int NW = T::NW, NT = 64 * NW;
   constexpr int KC = T::KC, NCK = KC / 8, NPC = T::NPC, NCH = T::EU / KC, SPC = KC / 16;
   constexpr int U = UT_<QT>::U, NP = U / 16;
+  constexpr int TL = pq_waves<QT, GU>() == 3 ? 1 : 2;    // 32-token tiles whose dots are live at a time
   constexpr int SPS = Q::SBW / 16;                       // K16 steps per sub-block
   constexpr int NXS = KC / 32, NSM = Q::SWS ? KC / Q::SWS : 0;  // token factor rows per chunk
   constexpr uint32_t WROWS = 32 * NW;
@@ -954,15 +969,13 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pq(PqArgs a) {
     }
   };
 
-  f32x16 acc[2][2], P[2][2];
+  f32x16 acc[2][2], zero;
+#pragma unroll
+  for (int r = 0; r < 16; r++) zero[r] = 0.0f;
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = P[i][j][r] = 0.0f;
-  const f32x16 zero = acc[0][0];
-  const bool two = m > 32;  // the second 32-token tile holds tokens
+    for (int j = 0; j < 2; j++) acc[i][j] = zero;
 
   if (u0 < u1) stage(u0, std::integral_constant<int, 0>{}, 0);
   __builtin_amdgcn_s_waitcnt(0);
@@ -980,32 +993,41 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pq(PqArgs a) {
       const uint8_t* xb = wb + WBYTES;
       const float* tf = reinterpret_cast<const float*>(xb + XBYTES);
       asm volatile("" : "+v"(tsw));
-      static_for<SPC>([&](auto ss) {
-        constexpr int SL = decltype(ss)::value, S = C * SPC + SL;
-        half8 bw[2], ax[2];
+      static_for<SPC / SPS>([&](auto sc) {
+        // sub-block SB: its dots on SPS K16 steps, then its term for every (row, token), added in
+        // K order, TL token tiles at a time
+        constexpr int SL = decltype(sc)::value * SPS, SB = C * (SPC / SPS) + decltype(sc)::value;
+        constexpr int EX = SL * 16 / 32, ES = Q::SWS ? SL * 16 / (Q::SWS ? Q::SWS : 1) : 0;
+        half8 bw[SPS][2];
+        static_for<SPS>([&](auto kc) {
+          constexpr int k = decltype(kc)::value;
 #pragma unroll
-        for (int rt = 0; rt < 2; rt++) bw[rt] = Q::template qfrag<C, S>(wb + row[rt], h);
-        const uint32_t pos = ((2 * SL + h) * 16) ^ tsw;
+          for (int rt = 0; rt < 2; rt++) bw[k][rt] = Q::template qfrag<C, C * SPC + SL + k>(wb + row[rt], h);
+        });
+        float rf[2][2];
 #pragma unroll
-        for (int tt = 0; tt < 2; tt++) ax[tt] = *reinterpret_cast<const half8*>(xb + xrow + pos + 32 * tt * NCK * 16);
+        for (int rt = 0; rt < 2; rt++) Q::template rowf<C, SB>(wb + row[rt], rf[rt]);
 #pragma unroll
-        for (int rt = 0; rt < 2; rt++) {
-          P[rt][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ax[0], bw[rt], S % SPS == 0 ? zero : P[rt][0], 0, 0, 0);
-          if (two)
-            P[rt][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ax[1], bw[rt], S % SPS == 0 ? zero : P[rt][1], 0, 0, 0);
-        }
-        if constexpr ((S + 1) % SPS == 0) {
-          // sub-block SB closes: its term for every (row, token), added in K order
-          constexpr int SB = S / SPS;
-          constexpr int EX = SL * 16 / 32, ES = Q::SWS ? SL * 16 / (Q::SWS ? Q::SWS : 1) : 0;
-          float rf[2][2];
+        for (int tl = 0; tl < 2; tl += TL) {
+          if (32 * tl >= (int)m) continue;
+          f32x16 P[TL][2];
 #pragma unroll
-          for (int rt = 0; rt < 2; rt++) Q::template rowf<C, SB>(wb + row[rt], rf[rt]);
+          for (int k = 0; k < SPS; k++) {
+            const uint32_t pos = ((2 * (SL + k) + h) * 16) ^ tsw;
 #pragma unroll
-          for (int tt = 0; tt < 2; tt++) {
+            for (int i = 0; i < TL; i++) {
+              if (32 * (tl + i) >= (int)m) continue;
+              const half8 ax = *reinterpret_cast<const half8*>(xb + xrow + pos + 32 * (tl + i) * NCK * 16);
+#pragma unroll
+              for (int rt = 0; rt < 2; rt++)
+                P[i][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ax, bw[k][rt], k == 0 ? zero : P[i][rt], 0, 0, 0);
+            }
+          }
+#pragma unroll
+          for (int tt = tl; tt < tl + TL; tt++) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-              if (32 * tt + 8 * j < m) {
+              if (32 * tt + 8 * j < (int)m) {
                 const uint32_t t4 = 32 * tt + 8 * j + 4 * h;
                 const float4 xs4 = *reinterpret_cast<const float4*>(tf + EX * kPfTok + t4);
                 float4 s4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -1016,9 +1038,15 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pq(PqArgs a) {
 #pragma unroll
                   for (int rt = 0; rt < 2; rt++) {
                     const int r = 4 * j + i;
-                    acc[rt][tt][r] = acc[rt][tt][r] + Q::term(P[rt][tt][r], rf[rt], xv[i], sv[i]);
+                    acc[rt][tt][r] = acc[rt][tt][r] + Q::term(P[tt - tl][rt][r], rf[rt], xv[i], sv[i]);
                   }
               }
+            }
+            // with one tile at a time its sums are pinned here, or the scheduler keeps several
+            // sub-blocks' dots live and spills (847 to 3052 VGPRs)
+            if constexpr (TL == 1) {
+#pragma unroll
+              for (int rt = 0; rt < 2; rt++) asm volatile("" : "+v"(acc[rt][tt]));
             }
           }
         }

@@ -93,6 +93,12 @@ def test_packed_prefill_many_tiles(dev):
 
 
 def test_packed_prefill_at_the_threshold(dev):
-    # 64 tokens of top-2 over 8 experts are 128 pairs: the smallest call k_pq takes,
-    # next to 63 tokens, which the decode kernels take
+    # 64 tokens of top-2 over 8 experts are 128 pairs, 16 an expert; next to 63 tokens
     check_layer(dev, 512, 512, 8, 2, (G.Q4_K,) * 3, (63, 64), G.MATH_PACKED, seed=81)
+
+
+@pytest.mark.parametrize("qts", [(G.Q4_K,) * 3, (G.Q3_K, G.Q3_K, G.Q4_K)])
+def test_packed_prefill_at_twelve_an_expert(dev, qts):
+    # 48 tokens of top-2 over 8 experts: 12 an expert, the smallest call of these types on
+    # k_pq, next to 47, which the decode kernels take
+    check_layer(dev, 512, 512, 8, 2, qts, (47, 48, 63), G.MATH_PACKED, seed=82)
