@@ -533,8 +533,9 @@ size_t plan_scratch(const Layer& L, uint32_t n, Carved* cv, uint8_t* base) {
   const bool h8 = uses_int8(L.math, L.p[2].qtype), pf = prefill_ok(D, n), pq = !pf && prefill_packed_ok(D, n);
   // prefill: hi and lo planes of the activations (f32 math) or one plane of their codes
   // and the transposed per-token scales and sums (packed math, nkp slots a row), hi and
-  // lo planes of h (both)
+  // lo planes of h (where k_pf takes the down product)
   const uint64_t nk_pf = (pf || pq) ? 2 * nk : 0, ns8 = h8 ? ns : 0, ns32 = h8 ? 0 : ns;
+  const uint64_t nk_h = pf || (pq && packed_down_pf(D, n)) ? 2 * nk : 0;
   const uint64_t nkp = pq ? nk + 64 : 0;
   size_t o_hs = P.add((size_t)n * L.d * 4), o_out = P.add((size_t)n * L.d * 4);
   size_t o_lin = P.add((size_t)n * L.ne * 4);
@@ -548,9 +549,8 @@ size_t plan_scratch(const Layer& L, uint32_t n, Carved* cv, uint8_t* base) {
   size_t o_cand = P.add((size_t)n * L.ne * 4);
   size_t o_work = P.add((size_t)L.ne * sizeof(ExpertWork));
   const uint32_t pcap = (pf || pq) ? prefill_tiles_cap(n, L.k, L.ne) : 0;
-  size_t o_pt = P.add((size_t)pcap * 4), o_xh = P.add(nk_pf * L.d * 2), o_hh = P.add(nk_pf * L.f * 2);
-  const uint64_t nk_sh = (pf || pq) ? 2 * nk : 0;
-  size_t o_xsh = P.add(nk_sh * (L.d / 16) * 2), o_hsh = P.add(nk_sh * (L.f / 16) * 2);
+  size_t o_pt = P.add((size_t)pcap * 4), o_xh = P.add(nk_pf * L.d * 2), o_hh = P.add(nk_h * L.f * 2);
+  size_t o_xsh = P.add(nk_pf * (L.d / 16) * 2), o_hsh = P.add(nk_h * (L.f / 16) * 2);
   size_t o_qxs = P.add(nkp * (L.d / 32) * 4), o_qxm = P.add(nkp * (L.d / 16) * 4);
   if (cv && base) {
     FwdBufs& B = cv->B;
@@ -644,12 +644,14 @@ gmoe_status run_layer(gmoe_ctx* c, Layer& L, FwdBufs B, uint32_t n, hipStream_t 
   }
   const bool quant = uses_int8(L.math, L.p[0].qtype);
   // prefill-sized calls run the expert products on MFMA over token tiles: f32 math
-  // (k_pf) or packed math (k_pq)
+  // (k_pf) or packed math (k_pq, then k_pf or the int8 down kernels)
   const bool pf = prefill_ok(D, n), pq = !pf && prefill_packed_ok(D, n);
+  const bool pf_down = pf || (pq && packed_down_pf(D, n));
   if (!pf && !pq) {
     B.ptile = nullptr;
-    B.xh = B.xsh = B.hh = B.hsh = nullptr;
+    B.xh = B.xsh = nullptr;
   }
+  if (!pf_down) B.hh = B.hsh = nullptr;
   if (!pq) B.qxs = B.qxsum = nullptr;
   // decode calls that compute their router logits: the expert products start on the
   // candidate experts, and the exact routing rides along in the gate/up launch. Any
@@ -706,7 +708,7 @@ gmoe_status run_layer(gmoe_ctx* c, Layer& L, FwdBufs B, uint32_t n, hipStream_t 
   }
   if (pf) HIP_TRY(launch_gather_f16(D, B, n, st));
   if (pq) HIP_TRY(launch_gather_codes(D, B, n, st));
-  const uint32_t ksg = (pf || pq) ? prefill_ksg(D, B) : down_ksg(D, n * L.k);
+  const uint32_t ksg = pf_down ? prefill_ksg(D, B) : down_ksg(D, n * L.k);
   Timing tm{};
   timed = timed && c->timing;
   if (timed) {  // no timing events inside a graph being captured
@@ -719,11 +721,11 @@ gmoe_status run_layer(gmoe_ctx* c, Layer& L, FwdBufs B, uint32_t n, hipStream_t 
   }
   HIP_TRY(pf ? launch_prefill_gateup(D, B, n, st) : pq ? launch_pq_gateup(D, B, n, st) : launch_gateup(D, B, n, ra, st));
   if (timed) HIP_TRY(hipEventRecord(tm.b, st));
-  // packed prefill: the down product's input is the dequantised h (scale * q), whose
-  // products k_pf makes exact; the down output is not requantised, so its summation order
-  // is free (outputs within rtol 1e-3 / atol 1e-4)
-  HIP_TRY((pf || pq) ? launch_prefill_down(D, B, n, ksg, st)
-                     : fuse ? launch_down_atomic(D, B, n, st) : launch_down(D, B, n, st));
+  // packed prefill on k_pf: the down product's input is the dequantised h (scale * q) as
+  // fp16 pairs; the down output is not requantised, so its summation order is free (outputs
+  // within rtol 1e-3 / atol 1e-4)
+  HIP_TRY(pf_down ? launch_prefill_down(D, B, n, ksg, st)
+                  : fuse ? launch_down_atomic(D, B, n, st) : launch_down(D, B, n, st));
   if (timed) {
     HIP_TRY(hipEventRecord(tm.c, st));
     c->pending.push_back(tm);

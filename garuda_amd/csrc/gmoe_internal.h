@@ -375,8 +375,10 @@ hipError_t launch_down_atomic(const LayerDev& L, const FwdBufs& B, uint32_t n, h
 bool prefill_ok(const LayerDev& L, uint32_t n);
 // Packed-math calls with enough tokens per expert run the products on MFMA: the
 // activation codes gathered in slot order, gate/up by k_pq (bit-exact h and codes), the
-// down product by k_pf on the dequantised h.
+// down product by k_pf on the dequantised h, or by the int8 kernels where packed_down_pf
+// says no.
 bool prefill_packed_ok(const LayerDev& L, uint32_t n);
+bool packed_down_pf(const LayerDev& L, uint32_t n);
 hipError_t launch_gather_codes(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st);
 hipError_t launch_pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st);
 bool prefill_dense_ok(const LayerDev& L, uint32_t n);

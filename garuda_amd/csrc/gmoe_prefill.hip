@@ -867,12 +867,18 @@ struct PqArgs {
   uint32_t nk, nkp, K, rows;
   uint32_t upk;         // dense: units of K per slice
   float* y;             // dense: [slices][nk][rows]
-  // h dequantised (scale * q of its int8 requantisation) as fp16 hi/lo planes [2][nk][rows],
-  // and its sums over swf rows as hi/lo planes [2][nk][rows/swf] (swf 0: none): the input
-  // of the f32-math down product (k_pf)
+  // gate/up: h requantised to int8, written for the down product that follows. For k_pf
+  // dequantised (scale * q) as fp16 hi/lo planes [2][nk][rows], with its sums over swf rows
+  // as hi/lo planes [2][nk][rows/swf] (swf 0: none). For the int8 down kernels (outf null)
+  // as quant_wave leaves it: codes [nk][rows], scales, sums in the down type's form.
   _Float16* outf;
   _Float16* outfs;
   uint32_t swf;
+  int8_t* hq;
+  float* hsc;
+  uint32_t* hsum;
+  int hkind;
+  int32_t hoff;
 };
 
 // Waves a SIMD of k_pq. The term's chain of VALU operations bounds it and two waves leave the
@@ -1072,6 +1078,14 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU>())) k_pq(Pq
         // quant_wave's arithmetic (quant/mod.rs:331-345)
         const uint32_t fr = bx * WROWS + 32 * wave + l32;
         const float hv = swiglu(acc[0][tt][r], acc[1][tt][r]);
+        if (!a.outf) {
+          // quant_wave's lanes 32.. write 32 rows after lanes ..31; here they are the same
+          // rows of another token, hence the h terms
+          const size_t sl = s0 + t;
+          quant_wave(hv, lane, t < m, a.hq + sl * a.rows + (fr - l32) - 32 * h, a.hsc + sl * (a.rows / 32) + (fr - l32) / 32 - h,
+                     a.hkind ? a.hsum + sl * (a.rows / sum_width(a.hkind)) : nullptr, fr - l32 - 32 * h, a.hkind, a.hoff);
+          continue;
+        }
         float am = fmaxf(0.0f, fabsf(hv));
 #pragma unroll
         for (int o = 16; o >= 1; o >>= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
@@ -1114,7 +1128,8 @@ uint32_t pf_rows(bool gu) {
   }
 }
 
-// The packed-math gate/up product (k_pq) of this block type; its down product is k_pf's.
+// The packed-math gate/up product (k_pq) of this block type; its down product is k_pf's, or
+// (B.hh null) the int8 down kernels'.
 template <int QT>
 hipError_t pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st) {
   if constexpr (!pq_type<QT>()) {
@@ -1134,6 +1149,11 @@ hipError_t pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_
     a.outf = B.hh;
     a.outfs = B.hsh;
     a.swf = pf_sum_width(L.qt_down);
+    a.hq = B.hq;
+    a.hsc = B.hsc;
+    a.hsum = B.hsum;
+    a.hkind = sum_kind_of(L.qt_down);
+    a.hoff = sum_offset_of(L.qt_down);
     hipLaunchKernelGGL((k_pq<QT, true>), dim3(L.f / pf_rows<QT>(true), B.ptile_cap), dim3(64 * PF<QT>::NW), 0, st, a);
     return hipGetLastError();
   }

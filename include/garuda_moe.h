@@ -61,7 +61,12 @@ enum { GMOE_COMBINE_EXPERT_ORDER = 0, GMOE_COMBINE_RANK_ORDER = 1 };
  * (llama/mod.rs:175-193 -> quant::matmul, quant/mod.rs:223-304): activations are
  * quantised to int8 per 32 and dotted with the packed rows for Q8_0 and Q2_K..Q6_K;
  * Q4_0/F16/F32 dequantise. F32 is Weight::Full under `mmap = false`
- * (llama/mod.rs:376-381 -> simd::matmul): every weight is the exact dequantised f32. */
+ * (llama/mod.rs:376-381 -> simd::matmul): every weight is the exact dequantised f32.
+ * Calls whose products run on MFMA as fp16 pairs (F32 math from 64 (token, expert) pairs and
+ * 4 an expert on; PACKED math's down product from 64 pairs and 16 an expert on; F32 dense
+ * calls from 64 tokens on) hold the product's input as the sum of two fp16 values: it, and
+ * its sums of 16 or 32 neighbours, must be below 65504 in magnitude, and below about 1e-3 it
+ * is held to 2^-25 absolute rather than to 22 bits. The other calls have the range of f32. */
 enum { GMOE_MATH_PACKED = 0, GMOE_MATH_F32 = 1 };
 
 /* Expert tensor layout (llama/mod.rs:223-226): one stacked `..._exps` tensor with

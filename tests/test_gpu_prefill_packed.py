@@ -102,3 +102,30 @@ def test_packed_prefill_at_twelve_an_expert(dev, qts):
     # 48 tokens of top-2 over 8 experts: 12 an expert, the smallest call of these types on
     # k_pq, next to 47, which the decode kernels take
     check_layer(dev, 512, 512, 8, 2, qts, (47, 48, 63), G.MATH_PACKED, seed=82)
+
+
+@pytest.mark.parametrize("qts", [(G.Q4_K,) * 3, (G.Q3_K, G.Q3_K, G.Q4_K), (G.Q3_K, G.Q3_K, G.Q2_K),
+                                 (G.Q4_K, G.Q4_K, G.Q6_K), (G.Q4_K, G.Q4_K, G.Q8_0)])
+@pytest.mark.parametrize("scale", [400.0, 1.0, 1e-3])
+def test_packed_calls_below_sixteen_an_expert_keep_the_range_of_h(dev, qts, scale):
+    # 12 to 15 tokens an expert: gate/up on k_pq, the down product on the int8 kernels, whose
+    # codes and f32 scales carry any h (fp16 pairs hold |h| below 65504 and lose bits of small
+    # ones). h is about scale^2: above 1e5 and near 1e-6 at the ends. gate/up is exact, so only
+    # the down product's f32 sums, in another order, differ: a few 1e-7 of the outputs' size.
+    d, f, ne, k = 512, 512, 8, 2
+    rng = np.random.default_rng(83)
+    gate, up = (M.quantize(qts[0], rng.normal(0, 0.05, ne * f * d).astype(np.float32)) for _ in range(2))
+    down = M.quantize(qts[2], rng.normal(0, 0.05, ne * f * d).astype(np.float32))
+    router = rng.normal(0, 0.02 / scale, ne * d).astype(np.float32)
+    layer = G.MoeLayer(dev, d, f, ne, k, router, gate, up, down, qts, math=G.MATH_PACKED)
+    L = dict(d=d, f=f, ne=ne, k=k, gating=0, combine=0, packed=1, router=router, qtypes=qts, gate=gate, up=up, down=down)
+    try:
+        for n in (48, 63):
+            say(f"packed {qts}, n={n}, activations x {scale}")
+            hs = (scale * rng.normal(0, 1, (n, d))).astype(np.float32)
+            out, ids, _ = layer.feed_forward_batch(hs)
+            want, wids, _ = O.feed_forward_batch(L, hs, threads=8)
+            assert np.array_equal(ids, wids)
+            assert np.abs(out - want).max() <= 2e-6 * np.abs(want).max()
+    finally:
+        layer.release()
