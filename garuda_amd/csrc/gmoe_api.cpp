@@ -526,16 +526,17 @@ bool uses_int8(uint32_t math, uint32_t qt);
 // The scratch of one launch sequence of n tokens: plan (base null) or carve. Buffers a
 // call of this size does not use take no room: h is int8 (packed math into an int8
 // down product) or f32, and only MFMA-prefill calls have token tiles and fp16 planes.
-size_t plan_scratch(const Layer& L, uint32_t n, Carved* cv, uint8_t* base) {
+// pf, pq: the call's route (run_layer).
+size_t plan_route(const Layer& L, uint32_t n, bool pf, bool pq, Carved* cv, uint8_t* base) {
   ScratchPlan P;
-  const uint64_t nk = (uint64_t)n * L.k, ns = slot_capacity(L, n);
   const LayerDev D = layer_dev(L);
-  const bool h8 = uses_int8(L.math, L.p[2].qtype), pf = prefill_ok(D, n), pq = !pf && prefill_packed_ok(D, n);
+  const bool h8 = uses_int8(L.math, L.p[2].qtype), pq8 = pq && !packed_down_pf(D, n);
+  const uint64_t nk = (uint64_t)n * L.k, ns = pq8 ? nk : slot_capacity(L, n);
   // prefill: hi and lo planes of the activations (f32 math) or one plane of their codes
   // and the transposed per-token scales and sums (packed math, nkp slots a row), hi and
   // lo planes of h (where k_pf takes the down product)
   const uint64_t nk_pf = (pf || pq) ? 2 * nk : 0, ns8 = h8 ? ns : 0, ns32 = h8 ? 0 : ns;
-  const uint64_t nk_h = pf || (pq && packed_down_pf(D, n)) ? 2 * nk : 0;
+  const uint64_t nk_h = pf || (pq && !pq8) ? 2 * nk : 0;
   const uint64_t nkp = pq ? nk + 64 : 0;
   size_t o_hs = P.add((size_t)n * L.d * 4), o_out = P.add((size_t)n * L.d * 4);
   size_t o_lin = P.add((size_t)n * L.ne * 4);
@@ -589,6 +590,16 @@ size_t plan_scratch(const Layer& L, uint32_t n, Carved* cv, uint8_t* base) {
     B.nkp = (uint32_t)nkp;
   }
   return P.total;
+}
+
+// Packed calls on k_pq with the int8 down product need less than the decode kernels do
+// (no candidate slots) and are given as much: which sizes the allocation-free forward takes
+// then does not depend on where the line between the two routes lies.
+size_t plan_scratch(const Layer& L, uint32_t n, Carved* cv, uint8_t* base) {
+  const LayerDev D = layer_dev(L);
+  const bool pf = prefill_ok(D, n), pq = !pf && prefill_packed_ok(D, n);
+  const size_t need = plan_route(L, n, pf, pq, cv, base);
+  return pq && !packed_down_pf(D, n) ? std::max(need, plan_route(L, n, false, false, nullptr, nullptr)) : need;
 }
 
 gmoe_status ensure_scratch(gmoe_ctx* c, size_t bytes) {

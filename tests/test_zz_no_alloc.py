@@ -15,6 +15,7 @@ import pytest
 
 import garuda_amd as G
 from garuda_amd import _lib
+from tests.helpers import fast_random_blocks
 from tests.test_gpu_dense import _hip
 from tests.test_gpu_parity import make_layer, say
 
@@ -101,6 +102,34 @@ def test_noalloc_forward_matches_the_async_forward():
             out = B.alloc(big * d * 4)
             rc = lib.gmoe_ffn_forward_noalloc(dev.handle, layer.id, hs, None, big, out, None, None, None)
             assert rc == 2 and b"allocation-free" in lib.gmoe_last_error()
+        finally:
+            B.free()
+            layer.release()
+
+
+def test_noalloc_takes_every_size_that_the_decode_route_fits():
+    # 64 MiB holds the decode kernels' scratch up to 59 tokens at this shape; from 48 tokens on
+    # k_pq takes gate/up, and a call that fits must not be refused for it
+    d, f, ne, k = 4096, 4096, 8, 2
+    rng = np.random.default_rng(78)
+    router = rng.normal(0, 0.02, ne * d).astype(np.float32)
+    raw = np.resize(fast_random_blocks(G.Q4_K, 4096, 78), ne * f * d // 256 * 144)
+    lib, hip = _lib.lib(), _runtime()
+    B = Bufs(hip)
+    with G.Device(0, slab_bytes=1 << 30) as dev:
+        layer = G.MoeLayer(dev, d, f, ne, k, router, raw, raw, raw, (G.Q4_K,) * 3)
+        try:
+            hs = B.alloc(64 * d * 4, rng.normal(0, 1, (64, d)).astype(np.float32))
+            out = B.alloc(64 * d * 4)
+            for n in (47, 48, 55, 56, 57, 58, 59):
+                say(f"no-alloc forward at the limit, n={n}")
+                assert lib.gmoe_ffn_forward_noalloc(dev.handle, layer.id, hs, None, n, out, None, None, None) == 0, n
+                a = B.fetch(out, (n, d), np.float32)
+                assert lib.gmoe_ffn_forward_async(dev.handle, layer.id, hs, None, n, out, None, None, None) == 0
+                assert np.array_equal(a.view(np.uint32), B.fetch(out, (n, d), np.float32).view(np.uint32))
+            for n in (60, 63, 64):
+                rc = lib.gmoe_ffn_forward_noalloc(dev.handle, layer.id, hs, None, n, out, None, None, None)
+                assert rc == 2 and b"allocation-free" in lib.gmoe_last_error(), n
         finally:
             B.free()
             layer.release()
