@@ -784,7 +784,9 @@ LayerDev dense_dev(const Dense& W) {
 
 struct DenseCarve {
   FwdBufs B;
-  uint32_t ksg;
+  uint32_t ksg;   // K slices of the result in y
+  PqDense split;  // of a k_pq call over the ksg_pq slices
+  uint32_t ksg_pq;
   bool pf, pq, int8;
 };
 
@@ -798,9 +800,9 @@ size_t plan_dense(const gmoe_ctx* c, const Dense& W, uint32_t n, uint8_t* base, 
   const bool int8 = !pf && !pq && uses_int8(W.math, W.qtype);
   FwdBufs B{};
   B.nslot = n;
-  B.ptile_cap = pf || pq ? (n + kPfTok - 1) / kPfTok : 0;
+  B.ptile_cap = pf ? (n + kPfTok - 1) / kPfTok : 0;
   B.nkp = n + kPfTok;  // a token tile's kPfTok factors are always in bounds
-  const uint32_t ksg = pf || pq ? 0u : dense_ksg(D);  // MFMA: from the carved buffers below
+  const uint32_t ksg = pf ? 0u : dense_ksg(D);  // k_pf's: from the carved buffers below
   ScratchPlan P;
   const size_t nx = (size_t)n * W.cols;
   size_t o_work = P.add(sizeof(ExpertWork)), o_off = P.add(8), o_act = P.add(8), o_tok = P.add((size_t)n * 4),
@@ -831,7 +833,7 @@ size_t plan_dense(const gmoe_ctx* c, const Dense& W, uint32_t n, uint8_t* base, 
     B.offsets = (uint32_t*)(base + o_off);
     B.active = (uint32_t*)(base + o_act);
     B.slot_tok = (uint32_t*)(base + o_tok);
-    B.ptile = pf || pq ? (uint32_t*)(base + o_pt) : nullptr;
+    B.ptile = pf ? (uint32_t*)(base + o_pt) : nullptr;
     if (int8 && !fuse) {
       B.hq = (int8_t*)(base + o_q);
       B.hsc = (float*)(base + o_s);
@@ -850,13 +852,15 @@ size_t plan_dense(const gmoe_ctx* c, const Dense& W, uint32_t n, uint8_t* base, 
     if (n <= kDenseTab) {  // the precomputed tables: no setup launch
       B.work = W.work_tab + (n - 1);
       B.slot_tok = c->ident;
-      if (pf || pq) B.ptile = c->ident;
+      if (pf) B.ptile = c->ident;
     }
     out->B = B;
     out->pf = pf;
     out->pq = pq;
     out->int8 = int8;
-    out->ksg = pf ? prefill_ksg(D, B) : pq ? pq_dense_ksg(D, B) : ksg;
+    out->split = pq ? pq_dense_split(D, n, ksg) : PqDense{};
+    out->ksg_pq = ksg;
+    out->ksg = pf ? prefill_ksg(D, B) : out->split.fold ? 1 : ksg;
   }
   return P.total;
 }
@@ -875,7 +879,7 @@ gmoe_status run_dense(const Dense& W, const DenseCarve& cv, const float* x, uint
     HIP_TRY(launch_prefill_down(D, B, n, cv.ksg, st));
   } else if (cv.pq) {
     HIP_TRY(launch_quant_codes(D, B, x, n, st));
-    HIP_TRY(launch_pq_dense(D, B, n, cv.ksg, st));
+    HIP_TRY(launch_pq_dense(D, B, n, cv.ksg_pq, cv.split, st));
   } else {
     if (cv.int8 && B.hq) {
       HIP_TRY(launch_quant_act(x, n, W.cols, B.hq, B.hsc, B.hsum, W.qtype, st));

@@ -312,8 +312,15 @@ __host__ __device__ constexpr uint32_t pq_sum_width(uint32_t qt) {
   return (qt == Q4_K || qt == Q5_K) ? 32u : qt == Q2_K ? 16u : 0u;
 }
 template <int QT> hipError_t pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st);
-template <int QT> uint32_t pq_dense_slices(const LayerDev& L, const FwdBufs& B);
-template <int QT> hipError_t pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, hipStream_t st);
+// A packed-math dense call on k_pq: tokens a workgroup (32 or 64), and whether each adds all
+// K slices up (the result is then one slice).
+struct PqDense {
+  uint32_t tok;
+  bool fold;
+};
+template <int QT> PqDense pq_dense_split(const LayerDev& L, uint32_t n, uint32_t ksg);
+template <int QT>
+hipError_t pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, PqDense p, hipStream_t st);
 template <int QT> hipError_t prefill_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st);
 template <int QT> hipError_t prefill_down(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg,
                                           hipStream_t st);
@@ -382,12 +389,13 @@ bool packed_down_pf(const LayerDev& L, uint32_t n);
 hipError_t launch_gather_codes(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st);
 hipError_t launch_pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st);
 bool prefill_dense_ok(const LayerDev& L, uint32_t n);
-// Packed-math dense projections on MFMA (k_pq): whether a call takes them, their K slices,
-// the activations' codes and the product.
+// Packed-math dense projections on MFMA (k_pq): whether a call takes them, the activations'
+// codes and the product.
 bool pq_dense_ok(const LayerDev& L, uint32_t n);
-uint32_t pq_dense_ksg(const LayerDev& L, const FwdBufs& B);
 hipError_t launch_quant_codes(const LayerDev& L, const FwdBufs& B, const float* x, uint32_t n, hipStream_t st);
-hipError_t launch_pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, hipStream_t st);
+// ksg: dense_ksg's K slices
+PqDense pq_dense_split(const LayerDev& L, uint32_t n, uint32_t ksg);
+hipError_t launch_pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, PqDense p, hipStream_t st);
 hipError_t launch_dense_setup(ExpertWork* work, uint32_t* offsets, uint32_t* active, uint32_t* ptile,
                               uint32_t ptile_cap, uint32_t* slot_tok, const uint8_t* w, uint32_t n, hipStream_t st);
 hipError_t launch_gather_f16(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st);

@@ -1614,29 +1614,38 @@ hipError_t launch_pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hip
   return hipErrorInvalidValue;
 }
 
-// Tokens from which a packed-math dense call runs on MFMA. The decode kernels' time grows
-// with every 8 tokens, a token tile's hardly: two layers' q|k|v and o (Q4_K, 6144 and 4096
-// rows of 4096) take 83.7 us there and about 85 here at 16 tokens, 110 and 88.6 at 24, 227
-// and 131 at 64, 791 and 193 at 256; the head (Q6_K, 32000 rows) 132 and 96 at 24, 313 and
-// 166 at 64.
-constexpr uint32_t kPqDenseMin = 24;
-
-bool pq_dense_ok(const LayerDev& L, uint32_t n) {
-  return L.math == 0 && n >= kPqDenseMin && pq_type_rt(L.qt_down) && L.d % 256 == 0 && L.f % 256 == 0;
+// Tokens from which a packed-math dense call runs on MFMA. The decode kernels' time grows with
+// the tokens, by a step after every 8, and with the rows; k_pq's hardly does up to 32 tokens,
+// and is least for the types of 32-value sub-blocks. Both give a row the same bits, so the
+// line is one of time only. Decode kernels and k_pq, us, columns 4096:
+//   rows 4096:  Q4_K 17 tokens 22.2 and 21.0, Q5_K 22.4 and 22.8, Q8_0 23.8 and 21.5, Q2_K 29.1
+//               and 28.0; Q3_K 24 tokens 26.5 and 26.0, Q6_K 24 tokens 27.5 and 29.7, 32 35.3 and 33.9;
+//   rows 14336: 17 tokens Q4_K 62.7 and 34.1, Q3_K 64.7 and 45.3, Q6_K 79.2 and 80.0 (20 tokens 96.3
+//               and 80.3); rows 32000: Q6_K 17 tokens 96.4 and 87.4, 64 tokens 313 and 164;
+//   rows 1024:  Q4_K 24 tokens 21.1 and 21.5, 32 27.6 and 23.3; Q3_K 32 tokens 29.4 and 30.0, 40
+//               32.7 and 31.1; Q6_K 40 tokens 34.3 and 35.2.
+static uint32_t pq_dense_min(uint32_t qt, uint32_t rows) {
+  if (rows < 4096) return qt == Q6_K ? 48 : qt == Q3_K ? 40 : 32;
+  if (rows < 8192) return qt == Q6_K ? 32 : qt == Q3_K ? 24 : 17;
+  return 17;
 }
 
-uint32_t pq_dense_ksg(const LayerDev& L, const FwdBufs& B) {
+bool pq_dense_ok(const LayerDev& L, uint32_t n) {
+  return L.math == 0 && pq_type_rt(L.qt_down) && n >= pq_dense_min(L.qt_down, L.d) && L.d % 256 == 0 && L.f % 256 == 0;
+}
+
+PqDense pq_dense_split(const LayerDev& L, uint32_t n, uint32_t ksg) {
   switch (L.qt_down) {
-#define DN(T) case T: return pq_dense_slices<T>(L, B);
+#define DN(T) case T: return pq_dense_split<T>(L, n, ksg);
     DN(Q4_K) DN(Q5_K) DN(Q6_K) DN(Q3_K) DN(Q2_K) DN(Q8_0)
 #undef DN
   }
-  return 1;
+  return {32, false};
 }
 
-hipError_t launch_pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, hipStream_t st) {
+hipError_t launch_pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, PqDense p, hipStream_t st) {
   switch (L.qt_down) {
-#define DN(T) case T: return pq_dense<T>(L, B, n, ksg, st);
+#define DN(T) case T: return pq_dense<T>(L, B, n, ksg, p, st);
     DN(Q4_K) DN(Q5_K) DN(Q6_K) DN(Q3_K) DN(Q2_K) DN(Q8_0)
 #undef DN
   }

@@ -712,8 +712,8 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pf(PfArgs a) {
 // Inputs: the activation codes in slot order as fp16 ([nk][K]), and the per-token
 // factors transposed, [K/32][nkp] scales and [K/SW][nkp] sums (nkp >= nk + 64 so a
 // token tile's 64 slots are always in bounds). Gate/up writes h's codes, scales and
-// sums the same way for the down product. A dense projection (k_pq<QT, false>) keeps the
-// terms in K order within a slice of K.
+// sums for the down product. A dense projection (k_pq<QT, false>) sums the terms as the decode
+// kernels do.
 // ---------------------------------------------------------------------------------
 template <int QT> struct PQ;
 
@@ -865,8 +865,8 @@ struct PqArgs {
   const float* ins;     // [K/32][nkp] activation scales
   const float* insum;   // [K/SWS][nkp] activation sums (types with SWS)
   uint32_t nk, nkp, K, rows;
-  uint32_t upk;         // dense: units of K per slice
-  float* y;             // dense: [slices][nk][rows]
+  uint32_t ksg;         // dense: K slices
+  float* y;             // dense: [ksg][nk][rows], or [nk][rows] where one workgroup takes them all
   // gate/up: h requantised to int8, written for the down product that follows. For k_pf
   // dequantised (scale * q) as fp16 hi/lo planes [2][nk][rows], with its sums over swf rows
   // as hi/lo planes [2][nk][rows/swf] (swf 0: none). For the int8 down kernels (outf null)
@@ -885,48 +885,58 @@ struct PqArgs {
 // SIMD waiting half the time, so gate/up takes three workgroups a CU where their LDS fits
 // (Q4_K, Q3_K, Q2_K), within 168 VGPRs: one 32-token tile's dots are live at a time. Zipf
 // tokens of the Mixtral shape, packed math: Q4_K 512 tokens 1195 -> 1094 us, 120 tokens 634
-// -> 542; Q3_K gate/up 1559 -> 1456 and 823 -> 734. Where three do not fit, and in a dense
-// call, whose K slices make two workgroups a CU, both tiles' dots are made before the
-// terms: the other order cost the Q6_K head at 64 tokens 166 -> 172 us.
-template <int QT, bool GU>
+// -> 542; Q3_K gate/up 1559 -> 1456 and 823 -> 734. Where three do not fit, both tiles' dots
+// are made before the terms.
+template <int QT, bool GU, int TOK>
 constexpr int pq_waves() {
   constexpr int KC = PF<QT>::KC;
-  constexpr int BUF = PF<QT>::NW * PF<QT>::NPC * 1024 + (int)kPfTok * (KC * 2 + 4 * (KC / 32 + (PQ<QT>::SWS ? KC / PQ<QT>::SWS : 0)));
-  return GU && 3 * 2 * BUF <= 160 * 1024 ? 3 : 2;
+  constexpr int BUF = PF<QT>::NW * PF<QT>::NPC * 1024 + TOK * (KC * 2 + 4 * (KC / 32 + (PQ<QT>::SWS ? KC / PQ<QT>::SWS : 0)));
+  return (GU || (TOK == 32 && PQ<QT>::SBW == 32)) && 3 * 2 * BUF <= 160 * 1024 ? 3 : 2 * 2 * BUF <= 160 * 1024 ? 2 : 1;
 }
 
-// GU: gate/up, the whole of K in one workgroup. !GU: a dense projection (rows of one
-// matrix, units [u0, u1) of K per blockIdx.z slice, output y slice blockIdx.z), tiled as
-// k_pf's down product.
-template <int QT, bool GU>
-__global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU>())) k_pq(PqArgs a) {
+// GU: gate/up, the whole of K in one workgroup. !GU: a dense projection: blockIdx.x NW * 64
+// rows of one matrix, blockIdx.y TOK tokens, blockIdx.z one of the decode kernels' a.ksg K
+// slices (k_dn_units's: kDnKS unit ranges, each summed in K order by itself, added in range
+// order), or gridDim.z = 1 and all of them, each added to the ones before it in y. A row's
+// output, its slices added in order, is then the decode kernels' bit for bit, whatever else
+// is in the batch.
+template <int QT, bool GU, int TOK>
+__global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU, TOK>())) k_pq(PqArgs a) {
   using T = PF<QT>;
   using Q = PQ<QT>;
   constexpr int NW = T::NW, NT = 64 * NW;
   constexpr int KC = T::KC, NCK = KC / 8, NPC = T::NPC, NCH = T::EU / KC, SPC = KC / 16;
   constexpr int U = UT_<QT>::U, NP = U / 16;
-  constexpr int TL = pq_waves<QT, GU>() == 3 ? 1 : 2;    // 32-token tiles whose dots are live at a time
+  constexpr int NTT = TOK / 32;                           // 32-token tiles
+  // tiles whose dots are live at a time
+  constexpr int TL = TOK == 32 || pq_waves<QT, GU, TOK>() == (GU ? 3 : 2) ? 1 : 2;
   constexpr int SPS = Q::SBW / 16;                       // K16 steps per sub-block
   constexpr int NXS = KC / 32, NSM = Q::SWS ? KC / Q::SWS : 0;  // token factor rows per chunk
   constexpr uint32_t WROWS = 32 * NW;
-  constexpr uint32_t WBYTES = NW * NPC * 1024, XBYTES = kPfTok * KC * 2, TBYTES = (NXS + NSM) * kPfTok * 4;
+  constexpr uint32_t WBYTES = NW * NPC * 1024, XBYTES = TOK * KC * 2, TBYTES = (NXS + NSM) * TOK * 4;
   constexpr uint32_t BUF = WBYTES + XBYTES + TBYTES;
-  constexpr int NX = (int)kPfTok * NCK / NT;              // activation loads per thread per chunk
-  static_assert(NX >= 1 && (int)kPfTok * NCK % NT == 0, "activation staging");
+  constexpr int NX = TOK * NCK / NT;                      // activation loads per thread per chunk
+  static_assert(NX >= 1 && TOK * NCK % NT == 0, "activation staging");
+  constexpr int FR = 64 / TOK;                            // token factor rows a wave loads at a time
+  static_assert((NXS + NSM) % FR == 0, "token factor rows");
   static_assert(2 * BUF <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(16))) uint8_t lds[2 * BUF];
 
   uint32_t bx = blockIdx.x, by = blockIdx.y;
   if constexpr (GU) pf_block(bx, by);
-  const uint32_t pt = a.ptile[by];
+  const uint32_t pt = GU ? a.ptile[by] : by;
   if (pt == ~0u) return;
-  const ExpertWork* W = a.work + (pt >> 16);
-  const uint32_t t0 = (pt & 0xffffu) * kPfTok;
-  const uint32_t m = min(kPfTok, W->m - t0), s0 = W->s0 + t0;
+  const ExpertWork* W = GU ? a.work + (pt >> 16) : a.work;
+  const uint32_t t0 = (GU ? pt & 0xffffu : pt) * TOK;
+  const uint32_t m = min((uint32_t)TOK, W->m - t0), s0 = W->s0 + t0;
   const uint32_t tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t K = a.K, nunit = K / T::EU;
-  const uint32_t u0 = GU ? 0 : blockIdx.z * a.upk, u1 = GU ? nunit : min(nunit, u0 + a.upk);
+  // the workgroup's unit ranges, q0 .. q1 - 1, and where range q starts
+  static_assert(kDnKS == 2, "two unit ranges a slice");
+  const uint32_t q0 = GU ? 0 : 2 * blockIdx.z, q1 = GU ? 1 : gridDim.z == 1 ? 2 * a.ksg : q0 + 2;
+  auto range = [&](uint32_t q) { return GU ? q * nunit : (nunit * q) / (2 * a.ksg); };
+  const uint32_t u0 = range(q0), u1 = range(q1);
 
   // GU: NW/2 gate tiles then NW/2 up tiles of 64 rows; wave w owns rows 32 (w % 2) .. of gate
   // tile w / 2 (rt = 0) and of the same up tile (rt = 1). !GU: NW tiles, wave w owns tile w
@@ -959,34 +969,64 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU>())) k_pq(Pq
 #pragma unroll
     for (int j = 0; j < NX; j++) {
       const uint32_t wq = NW * j + wave;
-      const uint32_t t = (RW * wq) % kPfTok + lane / NCK, c = (lane % NCK) ^ (t % NCK), tc = min(t, m - 1);
+      const uint32_t t = (RW * wq) % TOK + lane / NCK, c = (lane % NCK) ^ (t % NCK), tc = min(t, m - 1);
       lds_load16(a.in + ((size_t)(s0 + tc) * K + k0 + 8 * c), xb + 1024 * wq);
     }
-    // token factors: row r of the chunk (scales, then sums) = 64 floats of slots s0..
+    // token factors: row r of the chunk (scales, then sums) = TOK floats of slots s0..
 #pragma unroll
-    for (int j = 0; j < (NXS + NSM + NW - 1) / NW; j++) {
-      const uint32_t r = NW * j + wave;
-      if (r < (uint32_t)(NXS + NSM)) {
+    for (int j = 0; j < (NXS + NSM + FR * NW - 1) / (FR * NW); j++) {
+      const uint32_t rw = FR * (NW * j + wave), r = rw + lane / TOK;
+      if (rw < (uint32_t)(NXS + NSM)) {
         const float* src = r < (uint32_t)NXS ? a.ins + (size_t)(k0 / 32 + r) * a.nkp
                                              : a.insum + (size_t)(k0 / (Q::SWS ? Q::SWS : 1) + r - NXS) * a.nkp;
-        __builtin_amdgcn_global_load_lds(src + s0 + lane, (__attribute__((address_space(3))) void*)(tb + 256 * r), 4,
-                                         0, 0);
+        __builtin_amdgcn_global_load_lds(src + s0 + lane % TOK, (__attribute__((address_space(3))) uint8_t*)lds + (tb - lds) + TOK * 4 * rw,
+                                         4, 0, 0);
       }
     }
   };
 
-  f32x16 acc[2][2], zero;
+  f32x16 acc[2][NTT], first[2][NTT], zero;  // first: the sums of a dense slice's first range
 #pragma unroll
   for (int r = 0; r < 16; r++) zero[r] = 0.0f;
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++) acc[i][j] = zero;
+    for (int j = 0; j < NTT; j++) acc[i][j] = first[i][j] = zero;
+  // dense: a K slice's sums to slice sl of y, or added to what is there
+  auto write = [&](uint32_t sl, bool add) {
+    uint32_t c = l32, t0r = 4 * h;
+    asm volatile("" : "+v"(c), "+v"(t0r));  // the addresses are made here, not kept across the loop
+    float* y = a.y + (size_t)sl * a.nk * a.rows + (size_t)s0 * a.rows + bx * 64 * NW + 64 * wave + c;
+#pragma unroll
+    for (int tt = 0; tt < NTT; tt++) {
+      f32x16 v[2] = {first[0][tt] + acc[0][tt], first[1][tt] + acc[1][tt]};
+      if (add) {
+        f32x16 o[2];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const uint32_t t = min(32 * tt + 8 * (r / 4) + t0r + (r % 4), m - 1);
+#pragma unroll
+          for (int rt = 0; rt < 2; rt++) o[rt][r] = y[t * a.rows + 32 * rt];
+        }
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++) v[rt] = o[rt] + v[rt];
+      }
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const uint32_t t = 32 * tt + 8 * (r / 4) + t0r + (r % 4);
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+          if (t < m) y[t * a.rows + 32 * rt] = v[rt][r];
+      }
+    }
+  };
 
   if (u0 < u1) stage(u0, std::integral_constant<int, 0>{}, 0);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  for (uint32_t u = u0; u < u1; u++) {
+  uint32_t u = u0;
+  for (uint32_t q = q0; q < q1; q++) {
+  for (const uint32_t ue = range(q + 1); u < ue; u++) {
     static_for<NCH>([&](auto cc) {
       constexpr int C = decltype(cc)::value;
       const uint32_t b = (NCH % 2 == 0) ? (uint32_t)(C % 2) : ((u - u0) * NCH + C) % 2;
@@ -1014,7 +1054,7 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU>())) k_pq(Pq
 #pragma unroll
         for (int rt = 0; rt < 2; rt++) Q::template rowf<C, SB>(wb + row[rt], rf[rt]);
 #pragma unroll
-        for (int tl = 0; tl < 2; tl += TL) {
+        for (int tl = 0; tl < NTT; tl += TL) {
           if (32 * tl >= (int)m) continue;
           f32x16 P[TL][2];
 #pragma unroll
@@ -1035,9 +1075,9 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU>())) k_pq(Pq
             for (int j = 0; j < 4; j++) {
               if (32 * tt + 8 * j < (int)m) {
                 const uint32_t t4 = 32 * tt + 8 * j + 4 * h;
-                const float4 xs4 = *reinterpret_cast<const float4*>(tf + EX * kPfTok + t4);
+                const float4 xs4 = *reinterpret_cast<const float4*>(tf + EX * TOK + t4);
                 float4 s4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if constexpr (Q::SWS != 0) s4 = *reinterpret_cast<const float4*>(tf + (NXS + ES) * kPfTok + t4);
+                if constexpr (Q::SWS != 0) s4 = *reinterpret_cast<const float4*>(tf + (NXS + ES) * TOK + t4);
                 const float xv[4] = {xs4.x, xs4.y, xs4.z, xs4.w}, sv[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
                 for (int i = 0; i < 4; i++)
@@ -1061,19 +1101,26 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU>())) k_pq(Pq
       __syncthreads();
     });
   }
+  if constexpr (!GU) {
+    if (q % 2) write(blockIdx.z, q - q0 > 1);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < NTT; j++) {
+        first[i][j] = acc[i][j];
+        acc[i][j] = zero;
+      }
+  }
+  }
+  if constexpr (!GU) return;
 
   // epilogue
 #pragma unroll
-  for (int tt = 0; tt < 2; tt++)
+  for (int tt = 0; tt < NTT; tt++)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       const uint32_t t = 32 * tt + 8 * (r / 4) + 4 * h + (r % 4);
-      if constexpr (!GU) {
-        float* y = a.y + (size_t)blockIdx.z * a.nk * a.rows;
-#pragma unroll
-        for (int rt = 0; rt < 2; rt++)
-          if (t < m) y[(size_t)(s0 + t) * a.rows + bx * 64 * NW + 64 * wave + 32 * rt + l32] = acc[rt][tt][r];
-      } else {
+      if constexpr (GU) {
         // h = silu(g) * u, then quantised per 32 rows (the 32 lanes of this half) with
         // quant_wave's arithmetic (quant/mod.rs:331-345)
         const uint32_t fr = bx * WROWS + 32 * wave + l32;
@@ -1154,36 +1201,43 @@ hipError_t pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_
     a.hsum = B.hsum;
     a.hkind = sum_kind_of(L.qt_down);
     a.hoff = sum_offset_of(L.qt_down);
-    hipLaunchKernelGGL((k_pq<QT, true>), dim3(L.f / pf_rows<QT>(true), B.ptile_cap), dim3(64 * PF<QT>::NW), 0, st, a);
+    hipLaunchKernelGGL((k_pq<QT, true, kPfTok>), dim3(L.f / pf_rows<QT>(true), B.ptile_cap), dim3(64 * PF<QT>::NW), 0, st, a);
     return hipGetLastError();
   }
 }
 
-// K slices of the packed-math dense product: two workgroups a CU at once, as fit its LDS,
-// each slice keeping at least two units.
+// Tokens of a packed-math dense workgroup, and whether it folds the K slices. 64 tokens (types
+// of 16-value sub-blocks, whose decoding 32 tokens do not pay for: the Q6_K head at 64 tokens
+// 164 us, with 32 a workgroup 198) where the grid then still fills three quarters of the
+// chip; else 32, which fits three workgroups a CU with 32-value sub-blocks. Folded where the
+// tiles alone fill the chip, so that no slices are written (Q4_K, 4096 x 4096 at 2048 tokens
+// 267 us, in slices 289); below, a workgroup a slice (at 250 tokens 47.6, folded 118).
 template <int QT>
-uint32_t pq_dense_slices(const LayerDev& L, const FwdBufs& B) {
-  if constexpr (!pq_type<QT>()) {
-    return 1;
-  } else {
-    const uint32_t tiles = (L.d / pf_rows<QT>(false)) * B.ptile_cap, nunit = L.f / PF<QT>::EU;
-    const uint32_t ks = min(min((2 * 256 + tiles - 1) / tiles, max(1u, nunit / 2)), kMaxKsg);
-    const uint32_t upk = (nunit + ks - 1) / ks;
-    return (nunit + upk - 1) / upk;
+PqDense pq_dense_split(const LayerDev& L, uint32_t n, uint32_t ksg) {
+  PqDense p{32, false};
+  if constexpr (pq_type<QT>()) {
+    const uint32_t row_tiles = L.d / pf_rows<QT>(false), wide = row_tiles * ((n + 63) / 64);
+    uint32_t tiles = row_tiles * ((n + 31) / 32), slots = 256 * pq_waves<QT, false, 32>();
+    if (PQ<QT>::SBW == 16 && n > 32 && 4 * wide * ksg >= 3 * 256 * pq_waves<QT, false, 64>()) {
+      p.tok = 64;
+      tiles = wide;
+      slots = 256 * pq_waves<QT, false, 64>();
+    }
+    p.fold = tiles >= slots;
   }
+  return p;
 }
 
-// A dense projection in packed math: the reference's int8 dots and terms, in K order
-// within a slice.
+// A dense projection in packed math: the reference's int8 dots and terms, over ksg K slices
+// as k_dn_units cuts them.
 template <int QT>
-hipError_t pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, hipStream_t st) {
+hipError_t pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ksg, PqDense p, hipStream_t st) {
   if constexpr (!pq_type<QT>()) {
     return hipErrorNotSupported;
   } else {
     if (L.d % pf_rows<QT>(false) || L.f % PF<QT>::EU || ksg < 1 || ksg > kMaxKsg) return hipErrorInvalidValue;
     PqArgs a{};
     a.work = B.work;
-    a.ptile = B.ptile;
     a.in = B.xh;
     a.ins = B.qxs;
     a.insum = B.qxsum;
@@ -1191,11 +1245,17 @@ hipError_t pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ks
     a.nkp = B.nkp;
     a.K = L.f;
     a.rows = L.d;
-    const uint32_t nunit = L.f / PF<QT>::EU;
-    a.upk = (nunit + ksg - 1) / ksg;
+    a.ksg = ksg;
     a.y = B.y;
-    hipLaunchKernelGGL((k_pq<QT, false>), dim3(L.d / pf_rows<QT>(false), B.ptile_cap, ksg), dim3(64 * PF<QT>::NW), 0,
-                       st, a);
+    const dim3 grid(L.d / pf_rows<QT>(false), (n + p.tok - 1) / p.tok, p.fold ? 1 : ksg);
+    if constexpr (PQ<QT>::SBW == 16) {
+      if (p.tok == 64) {
+        hipLaunchKernelGGL((k_pq<QT, false, 64>), grid, dim3(64 * PF<QT>::NW), 0, st, a);
+        return hipGetLastError();
+      }
+    }
+    if (p.tok != 32) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_pq<QT, false, 32>), grid, dim3(64 * PF<QT>::NW), 0, st, a);
     return hipGetLastError();
   }
 }
@@ -1264,7 +1324,7 @@ template uint32_t prefill_down_slices<GMOE_QT>(const LayerDev&, const FwdBufs&);
 template hipError_t prefill_gateup<GMOE_QT>(const LayerDev&, const FwdBufs&, uint32_t, hipStream_t);
 template hipError_t prefill_down<GMOE_QT>(const LayerDev&, const FwdBufs&, uint32_t, uint32_t, hipStream_t);
 template hipError_t pq_gateup<GMOE_QT>(const LayerDev&, const FwdBufs&, uint32_t, hipStream_t);
-template uint32_t pq_dense_slices<GMOE_QT>(const LayerDev&, const FwdBufs&);
-template hipError_t pq_dense<GMOE_QT>(const LayerDev&, const FwdBufs&, uint32_t, uint32_t, hipStream_t);
+template PqDense pq_dense_split<GMOE_QT>(const LayerDev&, uint32_t, uint32_t);
+template hipError_t pq_dense<GMOE_QT>(const LayerDev&, const FwdBufs&, uint32_t, uint32_t, PqDense, hipStream_t);
 
 }  // namespace gmoe

@@ -214,9 +214,34 @@ def test_dense_refusals(dev):
 
 @pytest.mark.parametrize("qtype", [G.Q4_K, G.Q5_K, G.Q6_K, G.Q3_K, G.Q2_K, G.Q8_0])
 def test_dense_packed_on_mfma(dev, qtype):
-    # rows and columns a multiple of 256 from 24 tokens on: k_pq's dots, terms and slices, with
-    # half token tiles, ragged last ones, one unit a row and a call past the table of 2048
+    # rows and columns a multiple of 256, on both sides of pq_dense_min (32 to 48 tokens at so few
+    # rows): k_pq's dots, terms and slices, with half token tiles, ragged last ones, one unit a row and a call past the table of 2048
     check(dev, qtype, 256, 256, (23, 24, 33, 63, 65, 130), G.MATH_PACKED, seed=5)
     check(dev, qtype, 768, 1792, (32, 97), G.MATH_PACKED, seed=6)
     if qtype == G.Q4_K:
         check(dev, qtype, 256, 512, (2048, 2049), G.MATH_PACKED, seed=7)
+
+
+@pytest.mark.parametrize("qtype,rows,cols,ns", [
+    # 16 tokens and fewer run the decode kernels, these k_pq in its forms: half-full and ragged tiles
+    # of 32, 64 tokens a workgroup (16-value sub-blocks on full grids), slices of uneven unit ranges,
+    # one slice, one unit a row, the K slices folded in one workgroup
+    (G.Q4_K, 4096, 1792, (17, 33, 250)), (G.Q5_K, 4096, 1024, (17, 64)), (G.Q8_0, 4096, 2304, (23, 130)),
+    (G.Q2_K, 4096, 1536, (17, 250)), (G.Q3_K, 4096, 4096, (24, 250)), (G.Q6_K, 4096, 4096, (33, 129)),
+    (G.Q4_K, 256, 256, (32, 97)), (G.Q3_K, 768, 512, (41, 300)), (G.Q6_K, 512, 2816, (48, 65)),
+    (G.Q4_K, 256, 1024, (24577,)), (G.Q6_K, 16384, 768, (65, 256)), (G.Q2_K, 8192, 1024, (1025,))])
+def test_dense_packed_rows_do_not_depend_on_the_batch(dev, qtype, rows, cols, ns):
+    # a token's row has the same bits in a large batch as in one of at most 16 tokens
+    e, _ = O.block_layout(qtype)
+    W = G.DenseWeight(dev, qtype, rows, cols, fast_random_blocks(qtype, rows * cols // e, 41 + qtype), G.MATH_PACKED)
+    try:
+        for n in ns:
+            say(f"dense rows by batch {qtype} {rows}x{cols} n={n}")
+            xs = np.random.default_rng(n).normal(0, 1, (n, cols)).astype(np.float32)
+            xs[n // 2, :40] = 0.0
+            got = W.matmul_rows(xs)
+            at = sorted(set(range(min(n, 40))) | set(range(max(0, n - 70), n)) | set(range(0, n, 61)))
+            for i in range(0, len(at), 16):
+                assert np.array_equal(bits(got[at[i:i + 16]]), bits(W.matmul_rows(xs[at[i:i + 16]])))
+    finally:
+        W.release()
