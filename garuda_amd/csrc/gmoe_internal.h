@@ -311,6 +311,9 @@ __host__ __device__ constexpr uint32_t pf_sum_width(uint32_t qt) {
 __host__ __device__ constexpr uint32_t pq_sum_width(uint32_t qt) {
   return (qt == Q4_K || qt == Q5_K) ? 32u : qt == Q2_K ? 16u : 0u;
 }
+// Gate/up types that k_pq takes below the line of k_pf's down product (packed_down_pf): their h
+// then goes to the int8 down kernels.
+constexpr bool pq_int8_down(uint32_t qt) { return qt == Q4_K || qt == Q3_K; }
 template <int QT> hipError_t pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_t st);
 // A packed-math dense call on k_pq: tokens a workgroup (32 or 64), and whether each adds all
 // K slices up (the result is then one slice).

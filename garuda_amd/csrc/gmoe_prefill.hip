@@ -869,7 +869,7 @@ struct PqArgs {
   float* y;             // dense: [ksg][nk][rows], or [nk][rows] where one workgroup takes them all
   // gate/up: h requantised to int8, written for the down product that follows. For k_pf
   // dequantised (scale * q) as fp16 hi/lo planes [2][nk][rows], with its sums over swf rows
-  // as hi/lo planes [2][nk][rows/swf] (swf 0: none). For the int8 down kernels (outf null)
+  // as hi/lo planes [2][nk][rows/swf] (swf 0: none). For the int8 down kernels
   // as quant_wave leaves it: codes [nk][rows], scales, sums in the down type's form.
   _Float16* outf;
   _Float16* outfs;
@@ -900,8 +900,10 @@ constexpr int pq_waves() {
 // order), or gridDim.z = 1 and all of them, each added to the ones before it in y. A row's
 // output, its slices added in order, is then the decode kernels' bit for bit, whatever else
 // is in the batch.
-template <int QT, bool GU, int TOK>
-__global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU, TOK>())) k_pq(PqArgs a) {
+// H8: h for the int8 down kernels, else for k_pf (a build each: one kernel with both took
+// 1.5 % longer on k_pf's calls).
+template <int QT, bool GU, int TOK, int WAVES = pq_waves<QT, GU, TOK>(), bool H8 = false>
+__global__ void __launch_bounds__(64 * PF<QT>::NW, WAVES) k_pq(PqArgs a) {
   using T = PF<QT>;
   using Q = PQ<QT>;
   constexpr int NW = T::NW, NT = 64 * NW;
@@ -909,7 +911,7 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU, TOK>())) k_
   constexpr int U = UT_<QT>::U, NP = U / 16;
   constexpr int NTT = TOK / 32;                           // 32-token tiles
   // tiles whose dots are live at a time
-  constexpr int TL = TOK == 32 || pq_waves<QT, GU, TOK>() == (GU ? 3 : 2) ? 1 : 2;
+  constexpr int TL = TOK == 32 || WAVES == (GU ? 3 : 2) ? 1 : 2;
   constexpr int SPS = Q::SBW / 16;                       // K16 steps per sub-block
   constexpr int NXS = KC / 32, NSM = Q::SWS ? KC / Q::SWS : 0;  // token factor rows per chunk
   constexpr uint32_t WROWS = 32 * NW;
@@ -1125,7 +1127,7 @@ __global__ void __launch_bounds__(64 * PF<QT>::NW, (pq_waves<QT, GU, TOK>())) k_
         // quant_wave's arithmetic (quant/mod.rs:331-345)
         const uint32_t fr = bx * WROWS + 32 * wave + l32;
         const float hv = swiglu(acc[0][tt][r], acc[1][tt][r]);
-        if (!a.outf) {
+        if constexpr (H8) {
           // quant_wave's lanes 32.. write 32 rows after lanes ..31; here they are the same
           // rows of another token, hence the h terms
           const size_t sl = s0 + t;
@@ -1201,7 +1203,27 @@ hipError_t pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_
     a.hsum = B.hsum;
     a.hkind = sum_kind_of(L.qt_down);
     a.hoff = sum_offset_of(L.qt_down);
-    hipLaunchKernelGGL((k_pq<QT, true, kPfTok>), dim3(L.f / pf_rows<QT>(true), B.ptile_cap), dim3(64 * PF<QT>::NW), 0, st, a);
+    const dim3 grid(L.f / pf_rows<QT>(true), B.ptile_cap), block(64 * PF<QT>::NW);
+    constexpr int W = pq_waves<QT, true, kPfTok>();
+    // Three waves a SIMD lose to two where the workgroups, about one token tile an expert up to
+    // 20 tokens an expert, take two rounds either way and fill the second of three a CU to a
+    // third at most: 8 experts of 14336 rows (896 workgroups), 64 tokens, Q4_K 431 us and 410, Q3_K 539 and 511;
+    // skewed loads 485 and 477, 608 and 593. 128 experts of 768 (768): 219 and 271.
+    bool two = false;
+    if constexpr (W == 3) {
+      const uint32_t wgs = grid.x * L.ne;
+      two = a.nk <= 20 * L.ne && wgs > 3 * 256 && wgs <= 4 * 256;
+    }
+    if (!B.hh) {
+      if constexpr (pq_int8_down(QT)) {
+        if (two) hipLaunchKernelGGL((k_pq<QT, true, kPfTok, 2, true>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_pq<QT, true, kPfTok, W, true>), grid, block, 0, st, a);
+        return hipGetLastError();
+      }
+      return hipErrorNotSupported;
+    }
+    if (two) hipLaunchKernelGGL((k_pq<QT, true, kPfTok, 2>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_pq<QT, true, kPfTok>), grid, block, 0, st, a);
     return hipGetLastError();
   }
 }

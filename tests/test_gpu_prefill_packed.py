@@ -104,6 +104,11 @@ def test_packed_prefill_at_twelve_an_expert(dev, qts):
     check_layer(dev, 512, 512, 8, 2, qts, (47, 48, 63), G.MATH_PACKED, seed=82)
 
 
+def test_packed_prefill_with_two_workgroups_a_cu(dev):
+    # 8 experts of 104 row blocks: 832 workgroups, which run two a CU up to 20 tokens an expert
+    check_layer(dev, 512, 13312, 8, 2, (G.Q4_K,) * 3, (48, 64, 80, 81), G.MATH_PACKED, seed=85)
+
+
 @pytest.mark.parametrize("qts", [(G.Q4_K,) * 3, (G.Q3_K, G.Q3_K, G.Q4_K), (G.Q3_K, G.Q3_K, G.Q2_K),
                                  (G.Q4_K, G.Q4_K, G.Q6_K), (G.Q4_K, G.Q4_K, G.Q8_0)])
 @pytest.mark.parametrize("scale", [400.0, 1.0, 1e-3])
