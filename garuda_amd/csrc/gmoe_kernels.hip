@@ -1500,19 +1500,21 @@ static bool pq_type_rt(uint32_t qt) {
 }
 
 // Tokens per expert from which k_pq beats the decode kernels' gate/up (whose cost grows with
-// every 8 tokens an expert gets, while a token tile's hardly does); the down product is the
-// int8 kernels' on both sides below 16. Mixtral shape, decode kernels and k_pq: Q4_K 48
-// tokens (12 an expert) 536 and 437 us, 63 tokens 691 and 485; Q3_K gate/up 48 tokens 518 and
-// 526, 63 tokens 681 and 570. 128 experts of 2048 x 768 at 12 an expert: Q4_K 259 and 218,
-// Q3_K 272 and 242; Q6_K, one workgroup a CU: 329 and 405 with k_pf's down, equal at 16.
-constexpr uint32_t pq_min_per_expert(uint32_t qt) { return qt == Q4_K || qt == Q3_K ? 12 : 16; }
+// every 8 tokens an expert gets, while a token tile's hardly does); below kPfDownPerExpert the
+// down product is the int8 kernels' on both sides, and the bits are the same. Decode kernels and
+// k_pq, Mixtral shape: Q4_K 32 tokens (8 an expert) 369 and 375 us, 36 tokens 436 and 396, 48
+// tokens 544 and 445; Q3_K gate/up 40 tokens 465 and 487, 44 tokens 528 and 500, 56 tokens 630 and
+// 552. 128 experts of 2048 x 768: Q4_K 8 an expert 342 and 335, 9 366 and 332; Q3_K 9 an expert 351
+// and 360, 11 397 and 372. Q6_K, one workgroup a CU: 329 and 405 at 12, equal at 16.
+constexpr uint32_t kPfDownPerExpert = 16;
+constexpr uint32_t pq_min_per_expert(uint32_t qt) {
+  return !pq_int8_down(qt) ? kPfDownPerExpert : qt == Q4_K ? 9 : 11;
+}
 
 // Tokens per expert from which a packed call's down product is k_pf's. It reads h as fp16
 // pairs (hi, lo) and so needs |h|, and each sum of 16 or 32 of h, below 65504, and below
 // about 1e-3 it loses bits of h; the int8 kernels have neither limit and stay below the line.
 // Q4_K at 48 tokens of the Mixtral shape: 437 us with the int8 down product, 393 with k_pf's.
-constexpr uint32_t kPfDownPerExpert = 16;
-
 bool packed_down_pf(const LayerDev& L, uint32_t n) { return n * L.k >= kPfDownPerExpert * L.ne; }
 
 bool prefill_packed_ok(const LayerDev& L, uint32_t n) {

@@ -99,21 +99,22 @@ def test_packed_prefill_at_the_threshold(dev):
 
 @pytest.mark.parametrize("qts", [(G.Q4_K,) * 3, (G.Q3_K, G.Q3_K, G.Q4_K)])
 def test_packed_prefill_at_twelve_an_expert(dev, qts):
-    # 48 tokens of top-2 over 8 experts: 12 an expert, the smallest call of these types on
-    # k_pq, next to 47, which the decode kernels take
+    # 36 tokens of top-2 over 8 experts (9 an expert) are the smallest call of Q4_K gate/up on
+    # k_pq, 44 (11 an expert) of Q3_K; one token fewer runs the decode kernels
     check_layer(dev, 512, 512, 8, 2, qts, (47, 48, 63), G.MATH_PACKED, seed=82)
+    check_layer(dev, 512, 512, 8, 2, qts, (35, 36, 43, 44), G.MATH_PACKED, seed=84)
 
 
 def test_packed_prefill_with_two_workgroups_a_cu(dev):
     # 8 experts of 104 row blocks: 832 workgroups, which run two a CU up to 20 tokens an expert
-    check_layer(dev, 512, 13312, 8, 2, (G.Q4_K,) * 3, (48, 64, 80, 81), G.MATH_PACKED, seed=85)
+    check_layer(dev, 512, 13312, 8, 2, (G.Q4_K,) * 3, (36, 64, 80, 81), G.MATH_PACKED, seed=85)
 
 
 @pytest.mark.parametrize("qts", [(G.Q4_K,) * 3, (G.Q3_K, G.Q3_K, G.Q4_K), (G.Q3_K, G.Q3_K, G.Q2_K),
                                  (G.Q4_K, G.Q4_K, G.Q6_K), (G.Q4_K, G.Q4_K, G.Q8_0)])
 @pytest.mark.parametrize("scale", [400.0, 1.0, 1e-3])
 def test_packed_calls_below_sixteen_an_expert_keep_the_range_of_h(dev, qts, scale):
-    # 12 to 15 tokens an expert: gate/up on k_pq, the down product on the int8 kernels, whose
+    # Below 16 tokens an expert: gate/up on k_pq, the down product on the int8 kernels, whose
     # codes and f32 scales carry any h (fp16 pairs hold |h| below 65504 and lose bits of small
     # ones). h is about scale^2: above 1e5 and near 1e-6 at the ends. gate/up is exact, so only
     # the down product's f32 sums, in another order, differ: a few 1e-7 of the outputs' size.
