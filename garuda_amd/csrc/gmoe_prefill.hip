@@ -22,8 +22,8 @@
 //
 // Work layout. The dispatch lists the call's token tiles (kPfTok = 64 tokens of one
 // expert, in slot order) in B.ptile; blockIdx.y is a token tile. A workgroup has PF<QT>::NW = 4
-// waves, each owning 32 rows: gate/up workgroups take NW * 32 rows of f (both matrices:
-// 128), down workgroups NW * 64 rows of d. Each wave owns two 32-row MFMA row tiles (gate and up of its 32 rows, or
+// waves (F16: pf_nw), each owning 32 rows: gate/up workgroups take NW * 32 rows of f (both
+// matrices: 128), down workgroups NW * 64 rows of d. Each wave owns two 32-row MFMA row tiles (gate and up of its 32 rows, or
 // two 32-row halves of its 64 down rows) and both 32-token tiles: 4 accumulators of 32x32,
 // plus 4 of partial block sums. Per chunk of K (PF<QT>::KC values: 64; 128 for Q6_K, 32 for
 // F16) the workgroup copies the chunk's raw 16-byte pieces of its rows (the
@@ -456,11 +456,18 @@ __device__ __forceinline__ void pf_block(uint32_t& bx, uint32_t& by) {
   }
 }
 
+// Waves of a k_pf workgroup. F16 keeps 8 in gate/up: its chunks hold few values and bytes in
+// flight bound it (8 experts of 4096 x 14336, 64 tokens: 623 us with 4, 535 with 8). In its
+// down product 8 win below 16 tokens an expert (32 tokens 570 us with 4, 533 with 8) and 4
+// above and in dense calls (4096 x 4096 at 2048 tokens 178 -> 163 us).
 template <int QT, bool GU>
-__global__ void __launch_bounds__(64 * PF<QT>::NW, 2) k_pf(PfArgs a) {
+constexpr int pf_nw() { return QT == F16 && GU ? 8 : PF<QT>::NW; }
+
+template <int QT, bool GU, int NW = pf_nw<QT, GU>()>
+__global__ void __launch_bounds__(64 * NW, 2) k_pf(PfArgs a) {
   using T = PF<QT>;
   using D = Dec<QT>;
-  constexpr int NW = T::NW, NT = 64 * NW;
+  constexpr int NT = 64 * NW;
   constexpr int KC = T::KC, NCK = KC / 8, NPC = T::NPC, NCH = T::EU / KC, SPC = KC / 16;
   constexpr int U = UT_<QT>::U, NP = U / 16;
   constexpr uint32_t WROWS = 32 * NW * (GU ? 1 : 2);    // rows of a workgroup
@@ -1173,7 +1180,7 @@ uint32_t pf_rows(bool gu) {
   if constexpr (QT == F32) {
     return 0;
   } else {
-    return 32u * PF<QT>::NW * (gu ? 1u : 2u);
+    return gu ? 32u * pf_nw<QT, true>() : 64u * pf_nw<QT, false>();
   }
 }
 
@@ -1299,8 +1306,8 @@ hipError_t prefill_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipSt
     a.out = B.hh;
     a.swo = pf_sum_width(L.qt_down);
     a.outs = a.swo ? B.hsh : nullptr;
-    hipLaunchKernelGGL((k_pf<QT, true>), dim3(L.f / pf_rows<QT>(true), B.ptile_cap), dim3(64 * PF<QT>::NW), 0, st,
-                       a);
+    hipLaunchKernelGGL((k_pf<QT, true>), dim3(L.f / pf_rows<QT>(true), B.ptile_cap), dim3(64 * pf_nw<QT, true>()), 0,
+                       st, a);
     return hipGetLastError();
   }
 }
@@ -1336,7 +1343,13 @@ hipError_t prefill_down(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_
     const uint32_t nunit = L.f / PF<QT>::EU;
     a.upk = (nunit + ksg - 1) / ksg;
     a.y = B.y;
-    hipLaunchKernelGGL((k_pf<QT, false>), dim3(L.d / pf_rows<QT>(false), B.ptile_cap, ksg), dim3(64 * PF<QT>::NW),
+    if constexpr (QT == F16) {
+      if (L.ne > 1 && L.d % 512 == 0 && a.nk < 16 * L.ne) {
+        hipLaunchKernelGGL((k_pf<QT, false, 8>), dim3(L.d / 512, B.ptile_cap, ksg), dim3(512), 0, st, a);
+        return hipGetLastError();
+      }
+    }
+    hipLaunchKernelGGL((k_pf<QT, false>), dim3(L.d / pf_rows<QT>(false), B.ptile_cap, ksg), dim3(64 * pf_nw<QT, false>()),
                        0, st, a);
     return hipGetLastError();
   }
