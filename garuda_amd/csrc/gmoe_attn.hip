@@ -489,10 +489,13 @@ __global__ void __launch_bounds__(256) k_attn_combine(AttnArgs a) {
 // One workgroup per (kv head, tile of 256 (token, query head) rows, split of the keys), 8
 // waves of 32 rows. The single-token kernels read a kv head's keys and values once for
 // every token; here a 32-key tile in LDS serves 256 rows. The products run on bf16 MFMA at
-// f32 precision: an f32 is the sum of three bf16 of 8 bits each (split3, exact), and of
-// the nine products of two such sums the six down to 2^-16 of the first are taken; the
-// three left out are below 2^-23 of it, an f32 product's own rounding. Six passes of
-// v_mfma_f32_32x32x16_bf16 take 3/8 of the cycles of v_mfma_f32_32x32x2_f32.
+// f32 precision: an f32 is the sum of three bf16 of 8 bits each (split_planes, exact), and of
+// the nine products of two such sums the six down to 2^-16 of the first are taken. Each plane
+// is rounded to nearest, so the second is at most 2^-8 of the value and the third 2^-16, of
+// either sign: the three products left out are at most 2^-23 of the first (typically a
+// tenth of that) and cancel over a sum. (Truncated planes left up to 2^-21 out, always of
+// the product's sign.) Six passes of v_mfma_f32_32x32x16_bf16 take 3/8 of the cycles of
+// v_mfma_f32_32x32x2_f32.
 //   S^T = K Q^T: A = the keys (row l % 32), B = the wave's queries, so lane l holds the
 //     scores of query l % 32 for keys 8 (r / 4) + 4 (l / 32) + r % 4, r = 0..15;
 //   O^T = V^T P^T: with those keys taken in that order, lane l's own 16 probabilities are
@@ -506,40 +509,42 @@ __global__ void __launch_bounds__(256) k_attn_combine(AttnArgs a) {
 // GFLOP in six passes. A 32-key tile takes 3.9 us where its MFMAs take 2.6 (8 waves); 6 us
 // of a call are its start (tile, pages, first keys, queries) and its partial rows. With f32
 // MFMA instead the same call took 54 us. Row sums: the tile's products are summed by
-// themselves, smallest planes first, then added to the row's in one rounding (error against
-// 64 bits 1.7e-7; 3e-7 with one long chain, 1.9e-7 in the single-token kernels).
+// themselves, smallest planes first, then added to the row's in one rounding (with one long
+// chain the error against 64 bits was 1.8 times as large).
 //
 // Non-finite input: 0 * inf and inf - inf make NaNs of what f32 products would leave alone
 // (keys beside a row's span, -inf scores), so a row that meets a non-finite score or ends
 // with a non-finite sum is marked and summed by itself (attn_serial).
+//
+// The softmax runs in base 2 (v_exp_f32 on scores scaled by log2 e). Against 64 bits, relative
+// (2-norm), single-token kernels and this one: 32 heads on 8 of 128, 17 tokens 1.05e-7 and 0.82e-7,
+// 256 tokens 1.62e-7 and 1.30e-7, 1500 tokens 1.85e-7 and 1.57e-7; 8 heads on 2 of 32 1.55e-7 and 1.38e-7
+// at 1500; queries 16 times as large (scores to about 100) 6.7e-7 and 5.9e-7.
 // ---------------------------------------------------------------------------------
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-// x = a + b + c, the upper halves of the three words: 8 significant bits each.
-__device__ __forceinline__ void split3(float x, uint32_t& a, uint32_t& b, uint32_t& c) {
-  a = __float_as_uint(x);
-  const float r = x - __uint_as_float(a & 0xffff0000u);
-  b = __float_as_uint(r);
-  c = __float_as_uint(r - __uint_as_float(b & 0xffff0000u));
+// Two f32 rounded to a pair of bf16, and back.
+__device__ __forceinline__ uint32_t bf_pair(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
-// The upper halves of lo and hi as a bf16 pair.
-__device__ __forceinline__ uint32_t bf_pair(uint32_t lo, uint32_t hi) {
-  return __builtin_amdgcn_perm(hi, lo, 0x07060302u);
-}
-// N values (even) as three planes of bf16 pairs.
+// N values (even) as three planes of bf16 pairs: each plane what is left of the value after
+// the ones before it (exact: 24 bits in three signed 8-bit parts), rounded to nearest.
 template <int N>
 __device__ __forceinline__ void split_planes(const float* x, uint32_t (*w)[N / 2]) {
 #pragma unroll
   for (int i = 0; i < N / 2; i++) {
-    uint32_t a0, b0, c0, a1, b1, c1;
-    split3(x[2 * i], a0, b0, c0);
-    split3(x[2 * i + 1], a1, b1, c1);
-    w[0][i] = bf_pair(a0, a1);
-    w[1][i] = bf_pair(b0, b1);
-    w[2][i] = bf_pair(c0, c1);
+    float lo = x[2 * i], hi = x[2 * i + 1];
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+      w[p][i] = bf_pair(lo, hi);
+      lo -= __uint_as_float(w[p][i] << 16);
+      hi -= __uint_as_float(w[p][i] & 0xffff0000u);
+    }
   }
 }
 __device__ __forceinline__ bf16x8 frag4(const uint32_t* w) {

@@ -176,16 +176,17 @@ def _prompt_calls(kv, seqs, sizes, q, k, v, per=None):
 
 
 @pytest.mark.parametrize("nh,nkv,hd,bs,window,sizes", [
-    (4, 1, 128, 16, 0, (17,)), (4, 1, 128, 16, 0, (32,)), (4, 1, 128, 16, 0, (33, 65)),  # tile edges: 32 tokens of 4 heads
+    (4, 1, 128, 16, 0, (17,)), (4, 1, 128, 16, 0, (32,)), (4, 1, 128, 16, 0, (33, 65)),  # tile edges: 64 tokens of 4 heads
     (8, 8, 64, 16, 0, (127, 129)), (6, 2, 96, 8, 0, (64, 43)), (16, 1, 32, 4, 0, (21, 9)),  # group 1, 3, 16
     (32, 8, 128, 16, 0, (300, 1)), (8, 2, 32, 16, 50, (200, 40)), (8, 2, 64, 5, 1, (70,)),  # windows, odd pages
     (4, 4, 128, 16, 0, (600,)), (7, 1, 64, 16, 129, (400,)),
 ])
 def test_prompt_tiles_equal_single_tokens(dev, nh, nkv, hd, bs, window, sizes):
-    # A call of several consecutive tokens runs tiles of 128 (token, head) rows on MFMA; the
+    # A call of several consecutive tokens runs tiles of 256 (token, head) rows on MFMA; the
     # same prompt in calls of at most 16 tokens runs the single-token kernels. Both are f32
     # softmax-weighted means of the values, so they differ by the rounding of the scores
-    # (hd products each) and of the sums over the span, relative to the largest value.
+    # (hd products each) and of the sums over the span, relative to the largest value: a bound
+    # on the worst case (what the tiles keep of f32 precision is the next test's matter).
     rng = np.random.default_rng(hd + nh + len(sizes))
     n = sum(sizes)
     q, k, v = (rng.normal(size=(n, w)).astype(np.float32) for w in (nh * hd, nkv * hd, nkv * hd))
@@ -207,6 +208,66 @@ def test_prompt_tiles_equal_single_tokens(dev, nh, nkv, hd, bs, window, sizes):
         err = np.abs(x - y).max()
         assert err <= bound, f"err {err} bound {bound}"
         assert np.sqrt(np.mean((x - y) ** 2)) <= 1e-6 * np.sqrt(np.mean(y ** 2)) + bound / 50
+
+
+def _attention64(nh, nkv, hd, window, q, k, v):
+    """One sequence's contexts in 64 bits, rope_theta 1 (every pair turned by its position)."""
+    n = len(q)
+    pos = np.arange(n)[:, None, None]
+    c, s = np.cos(pos.astype(np.float64)), np.sin(pos.astype(np.float64))
+
+    def rot(x, heads):
+        a = x.astype(np.float64).reshape(n, heads, hd // 2, 2)
+        return np.stack([a[..., 0] * c - a[..., 1] * s, a[..., 0] * s + a[..., 1] * c], -1).reshape(n, heads, hd)
+
+    qr, kr, vv = rot(q, nh), rot(k, nkv), v.astype(np.float64).reshape(n, nkv, hd)
+    i = np.arange(n)
+    seen = (i[None] <= i[:, None]) & ((window == 0) | (i[None] > i[:, None] - window))
+    out = np.empty((n, nh, hd))
+    for h in range(nh):
+        sc = np.where(seen, qr[:, h] @ kr[:, h * nkv // nh].T / np.sqrt(hd), -np.inf)
+        w = np.exp(sc - sc.max(1, keepdims=True))
+        out[:, h] = w @ vv[:, h * nkv // nh] / w.sum(1, keepdims=True)
+    return out.reshape(n, nh * hd)
+
+
+@pytest.mark.parametrize("nh,nkv,hd,n,window,qscale", [
+    (4, 1, 128, 40, 0, 1.0), (8, 2, 128, 600, 0, 1.0), (8, 2, 128, 300, 70, 4.0), (8, 2, 32, 500, 0, 1.0),
+    (4, 4, 64, 257, 0, 1.0), (6, 2, 96, 200, 0, 2.0)])
+def test_prompt_tiles_are_as_precise_as_single_tokens(dev, nh, nkv, hd, n, window, qscale):
+    # The tiles' products of three bf16 planes claim f32 precision: against the same attention
+    # in 64 bits they must be no further off than the single-token kernels, whose products are
+    # f32 (the maximum, one value of thousands, within twice theirs). Any of the six plane
+    # products left out shows: the smallest of them are 2^-16 of a product, 250 f32 roundings.
+    rng = np.random.default_rng(n + hd)
+    q, k, v = (rng.normal(size=(n, w)).astype(np.float32) for w in (nh * hd, nkv * hd, nkv * hd))
+    q *= np.float32(qscale)
+    kw = dict(max_positions=700, sliding_window=window, max_seqs=1, rope_theta=1.0)
+    say(f"tile precision nh={nh} nkv={nkv} hd={hd} n={n} window={window} q x {qscale}")
+    with KvCache(dev, 1, nh, nkv, hd, **kw) as A, KvCache(dev, 1, nh, nkv, hd, **kw) as B:
+        tiles = _prompt_calls(A, [A.open_seq()], [n], q, k, v)
+        single = _prompt_calls(B, [B.open_seq()], [n], q, k, v, per=16)
+    want = _attention64(nh, nkv, hd, window, q, k, v)
+    et, es = np.abs(tiles - want), np.abs(single - want)
+    say(f"  rms {np.sqrt((et ** 2).mean()):.2e} single {np.sqrt((es ** 2).mean()):.2e}, max {et.max():.2e} single {es.max():.2e}")
+    assert np.sqrt((et ** 2).mean()) <= 1.05 * np.sqrt((es ** 2).mean())
+    assert et.max() <= 2 * es.max()
+
+
+def test_prompt_tiles_round_to_both_sides(dev):
+    # values in [1, 2) make every product positive: planes cut off instead of rounded would make
+    # each sum too small, by about 2^-24 of itself on average; rounded ones cancel
+    nh, nkv, hd, n = 8, 2, 64, 512
+    rng = np.random.default_rng(11)
+    q, k = (rng.normal(size=(n, w)).astype(np.float32) for w in (nh * hd, nkv * hd))
+    v = (1 + rng.random(size=(n, nkv * hd))).astype(np.float32)
+    say("tile bias")
+    with KvCache(dev, 1, nh, nkv, hd, max_positions=512, max_seqs=1, rope_theta=1.0) as A:
+        got = _prompt_calls(A, [A.open_seq()], [n], q, k, v)
+    want = _attention64(nh, nkv, hd, 0, q, k, v)
+    bias = ((got - want) / want).mean()
+    say(f"  mean relative error {bias:.2e}")
+    assert abs(bias) <= 2.0 ** -27
 
 
 @pytest.mark.parametrize("what", ["nan value", "inf value", "nan key", "inf key", "nan query"])
