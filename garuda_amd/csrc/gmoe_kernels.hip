@@ -1402,7 +1402,8 @@ static bool prefill_type(uint32_t qt) {
 
 bool prefill_ok(const LayerDev& L, uint32_t n) {
   const uint32_t nk = n * L.k;
-  // rows: gate/up workgroups take up to 256 rows of f, down ones up to 512 of d
+  // rows: gate/up workgroups take up to 256 rows of f, down ones 256 of d (F16: 512). Other
+  // multiples of 256 of d stay on the decode kernels, whose f32 activations have no fp16 pair's range
   return L.math == 1 && nk >= kPfMinSlots && nk >= 4 * L.ne && L.qt_gate == L.qt_up && prefill_type(L.qt_gate) &&
          prefill_type(L.qt_down) && L.d % 512 == 0 && L.f % 256 == 0 && L.ne < 65536;
 }

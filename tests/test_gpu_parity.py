@@ -241,13 +241,22 @@ def test_front_end_64_experts(dev):
 
 
 # f32 math from kPfMinSlots = 64 slots runs the expert products on MFMA (exact fp16
-# products, f32 sums) over token tiles of 64; Zipf-skewed loads give the busiest expert several
-# tiles, the last one partial.
+# products, f32 sums) over token tiles of 64 where d is a multiple of 512 and f of 256 (the
+# 256-wide layer below keeps the decode kernels); Zipf-skewed loads give the busiest expert
+# several tiles, the last one partial.
 @pytest.mark.parametrize("qts", [(G.Q4_K,) * 3, (G.Q5_K,) * 3, (G.Q6_K,) * 3, (G.Q3_K, G.Q3_K, G.Q4_K),
                                  (G.Q2_K,) * 3, (G.Q8_0,) * 3, (G.Q6_K, G.Q6_K, G.Q8_0), (G.Q4_0,) * 3,
                                  (G.F16,) * 3])
 def test_prefill_every_type(dev, qts):
     check_layer(dev, 256, 512, 8, 2, qts, (32, 300), G.MATH_F32, seed=20 + qts[0], zipf=True)
+
+
+@pytest.mark.parametrize("qts", [(G.Q4_K,) * 3, (G.Q5_K,) * 3, (G.Q6_K,) * 3, (G.Q3_K, G.Q3_K, G.Q4_K),
+                                 (G.Q2_K,) * 3, (G.Q8_0,) * 3, (G.Q6_K, G.Q6_K, G.Q8_0), (G.Q4_0,) * 3,
+                                 (G.F16,) * 3])
+def test_prefill_every_type_on_mfma(dev, qts):
+    # 8 tokens an expert and more (F16's down product changes its workgroup at 16), ragged tiles
+    check_layer(dev, 512, 768, 8, 2, qts, (32, 63, 64, 300), G.MATH_F32, seed=22 + qts[0], zipf=True)
 
 
 @pytest.mark.parametrize("qts", [(G.Q4_K,) * 3, (G.Q6_K, G.Q6_K, G.Q8_0), (G.Q4_0,) * 3])
