@@ -514,7 +514,7 @@ __global__ void __launch_bounds__(256) k_attn_combine(AttnArgs a) {
 //
 // Non-finite input: 0 * inf and inf - inf make NaNs of what f32 products would leave alone
 // (keys beside a row's span, -inf scores), so a row that meets a non-finite score or ends
-// with a non-finite sum is marked and summed by itself (attn_serial).
+// with a non-finite sum is marked and summed by itself (attn_row).
 //
 // The softmax runs in base 2 (v_exp_f32 on scores scaled by log2 e). Against 64 bits, relative
 // (2-norm), single-token kernels and this one: 32 heads on 8 of 128, 17 tokens 1.05e-7 and 0.82e-7,
@@ -562,7 +562,7 @@ __device__ __forceinline__ f32x16 mfma_rest(const bf16x8* a, const bf16x8* b, f3
   return mfma_bf(a[0], b[1], c);
 }
 
-// A split's max may be a mark: a row for attn_serial (a NaN pattern no max can be).
+// A split's max may be a mark: a row for attn_row (a NaN pattern no max can be).
 constexpr uint32_t kMarkSerial = 0x7fc00001u;
 
 __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 64); }
@@ -805,67 +805,157 @@ __global__ void __launch_bounds__(512, 2) k_attn_tile(AttnArgs a) {
   }
 }
 
-// Columns d .. d + 3 of query head hh of token i, position by position: for the rows that
-// k_attn_tile marks, which is rare.
-__device__ __forceinline__ float4 attn_serial(const AttnArgs& a, uint32_t i, uint32_t hh, uint32_t d) {
+// attn_uniform's four columns from d on.
+__device__ float4 attn_uniform4(const AttnArgs& a, uint32_t i, uint32_t hh, uint32_t d) {
   const AttnEntry e = entry(a, i);
   const uint32_t kh = hh / (a.n_heads / a.n_kv);
-  const size_t voff = (size_t)a.bs * a.n_kv * a.hd;
-  const float* q = a.qr + ((size_t)i * a.n_heads + hh) * a.hd;
-  float M = -INFINITY, L = 0.0f, o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  bool uni = false;
+  const float u = fdiv(1.0f, (float)(e.pos + 1 - e.start));
+  const size_t voff = (size_t)a.bs * a.n_kv * a.hd + d;
+  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   for (uint32_t p = e.start; p <= e.pos; p++) {
-    const float* kr = key_row(a, e, p, kh);
-    float s = 0.0f;
-    for (uint32_t x = 0; x < a.hd; x++) s = fmaf(q[x], kr[x], s);
-    s *= a.scale;
-    uni |= s != s || s == INFINITY;
-    if (uni || s == -INFINITY) continue;
-    if (s > M) {
-      const float f = gm_expf(M - s);
-      L *= f;
-      for (int b = 0; b < 4; b++) o[b] *= f;
-      M = s;
-    }
-    const float pv = gm_expf(s - M);
-    L += pv;
-    for (int b = 0; b < 4; b++) o[b] = fmaf(pv, kr[voff + d + b], o[b]);
+    const float4 v = *reinterpret_cast<const float4*>(key_row(a, e, p, kh) + voff);
+    o = make_float4(o.x + v.x * u, o.y + v.y * u, o.z + v.z * u, o.w + v.w * u);
   }
-  if (uni || M == -INFINITY)
-    return make_float4(attn_uniform(a, i, hh, d), attn_uniform(a, i, hh, d + 1), attn_uniform(a, i, hh, d + 2),
-                       attn_uniform(a, i, hh, d + 3));
-  return make_float4(o[0] / L, o[1] / L, o[2] / L, o[3] / L);
+  return o;
 }
 
-// The splits of a tiled call merged: a thread per four columns of a (token, head) row.
-// A marked row, or one without any score above -inf, is summed by itself.
-__global__ void __launch_bounds__(256) k_attn_merge(AttnArgs a) {
-  const uint32_t rows = a.n * a.n_heads, q4 = a.hd / 4, g = blockIdx.x * 256 + threadIdx.x, row = g / q4, x = g % q4;
-  if (row >= rows) return;
-  const float2* ml = reinterpret_cast<const float2*>(a.part + (size_t)a.nchunk * rows * a.hd) + row;
-  const float4* po = reinterpret_cast<const float4*>(a.part) + (size_t)row * q4 + x;
-  float M = -INFINITY, L = 0.0f;  // M in units of log2
-  bool serial = false;
-  for (uint32_t c = 0; c < a.nchunk; c++) {
-    const float m = ml[(size_t)c * rows].x;
-    serial |= m != m;
-    M = fmaxf(M, m);
-  }
+// Row hh of token i by the whole workgroup, for the rows that k_attn_tile marks (non-finite
+// input): chunks of kAttnChunk positions as the single-token kernels cut them, scores four
+// threads a position, values a thread per (every q4-th position, float4 column x = t % q4),
+// in f32. sc [kAttnChunk], po [256] in LDS. Returns false where the softmax falls back to
+// uniform weights (a NaN or +inf score, or none above -inf), as soon as that is known;
+// otherwise threads x < q4 have the row's columns 4 x .. 4 x + 3 in w.
+__device__ bool attn_row(const AttnArgs& a, uint32_t i, uint32_t hh, float* sc, float4* po, float4& w) {
+  const AttnEntry e = entry(a, i);
+  const uint32_t t = threadIdx.x, lane = t & 63, hd = a.hd, q4 = hd / 4, ng = 256 / q4, g = t / q4, x = t % q4;
+  const uint32_t kh = hh / (a.n_heads / a.n_kv);
+  const size_t voff = (size_t)a.bs * a.n_kv * hd;
+  const float4* q = reinterpret_cast<const float4*>(a.qr + ((size_t)i * a.n_heads + hh) * hd);
+  float M = -INFINITY, L = 0.0f;
   float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll 4
-  for (uint32_t c = 0; c < a.nchunk; c++) {
-    const float2 v = ml[(size_t)c * rows];
-    if (!(v.x > -INFINITY)) continue;  // nothing was written for an empty split
-    const float f = __builtin_amdgcn_exp2f(v.x - M);
-    const float4 p = po[(size_t)c * rows * q4];
-    L = fmaf(v.y, f, L);
-    o.x = fmaf(p.x, f, o.x);
-    o.y = fmaf(p.y, f, o.y);
-    o.z = fmaf(p.z, f, o.z);
-    o.w = fmaf(p.w, f, o.w);
+  for (uint32_t p0 = e.start; p0 <= e.pos; p0 += kAttnChunk) {
+    const uint32_t cnt = min(kAttnChunk, e.pos + 1 - p0), j = t >> 2;
+    float s = 0.0f;
+    if (j < cnt) {
+      const float4* kr = reinterpret_cast<const float4*>(key_row(a, e, p0 + j, kh));
+      for (uint32_t c = t & 3; c < q4; c += 4) {
+        const float4 kv = kr[c], qv = q[c];
+        s = fmaf(kv.x, qv.x, s);
+        s = fmaf(kv.y, qv.y, s);
+        s = fmaf(kv.z, qv.z, s);
+        s = fmaf(kv.w, qv.w, s);
+      }
+    }
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    if ((t & 3) == 0) sc[j] = j < cnt ? s * a.scale : -INFINITY;
+    __syncthreads();
+    const float v = sc[lane];
+    if (__ballot(v != v || v == INFINITY)) return false;  // every wave sees the same scores
+    const float mc = wave_max(v);
+    if (mc > -INFINITY) {  // a chunk without a score above -inf adds nothing
+      const float mn = fmaxf(M, mc), f = gm_expf(M - mn), pv = lane < cnt ? gm_expf(v - mn) : 0.0f;
+      M = mn;
+      L = fmaf(L, f, wave_sum(pv));
+      __syncthreads();
+      if (t < kAttnChunk) sc[t] = pv;
+      __syncthreads();
+      o = make_float4(o.x * f, o.y * f, o.z * f, o.w * f);
+      if (g < ng)
+        for (uint32_t jj = g; jj < cnt; jj += ng) {
+          const float4 vv = *reinterpret_cast<const float4*>(key_row(a, e, p0 + jj, kh) + voff + 4 * x);
+          const float pj = sc[jj];
+          o = make_float4(fmaf(pj, vv.x, o.x), fmaf(pj, vv.y, o.y), fmaf(pj, vv.z, o.z), fmaf(pj, vv.w, o.w));
+        }
+    }
+    __syncthreads();
   }
-  float4 w = make_float4(o.x / L, o.y / L, o.z / L, o.w / L);
-  if (serial || M == -INFINITY) w = attn_serial(a, row / a.n_heads, row % a.n_heads, 4 * x);
+  if (M == -INFINITY) return false;
+  po[t] = o;
+  __syncthreads();
+  if (t < q4) {
+    for (uint32_t k = 1; k < ng; k++) {
+      const float4 b = po[k * q4 + t];
+      o = make_float4(o.x + b.x, o.y + b.y, o.z + b.z, o.w + b.w);
+    }
+    w = make_float4(o.x / L, o.y / L, o.z / L, o.w / L);
+  }
+  return true;
+}
+
+// The splits of a tiled call merged: a thread per four columns of a (token, head) row, the
+// splits kIn at a time with a running max. Marked rows, and those without any score above
+// -inf, are then summed by the workgroup one after another (attn_row), the uniform ones of
+// them by their own threads: 256 tokens over a NaN key 128 tokens in 547 us, in the
+// single-token kernels 860 to 1100 (each thread summing its columns' row took 7.2 ms). With
+// many splits (40 tokens at 4000, 8 heads on 2 of 32: 63) a batch's loads are in flight
+// together: the call 54.5 -> 26 us.
+__global__ void __launch_bounds__(256) k_attn_merge(AttnArgs a) {
+  __shared__ float4 po[256];
+  __shared__ float sc[kAttnChunk];
+  __shared__ uint32_t marks;
+  const uint32_t rows = a.n * a.n_heads, q4 = a.hd / 4, rpb = 256 / q4, r = threadIdx.x / q4, x = threadIdx.x % q4;
+  const uint32_t row = blockIdx.x * rpb + r;
+  const bool mine = r < rpb && row < rows;
+  float4 w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  bool serial = false;
+  if (threadIdx.x == 0) marks = 0;
+  __syncthreads();
+  if (mine) {
+    constexpr uint32_t kIn = 8;
+    const float2* ml = reinterpret_cast<const float2*>(a.part + (size_t)a.nchunk * rows * a.hd) + row;
+    const float4* po4 = reinterpret_cast<const float4*>(a.part) + (size_t)row * q4 + x;
+    float M = -INFINITY, L = 0.0f;  // M in units of log2
+    float4 o = w;
+    for (uint32_t c0 = 0; c0 < a.nchunk; c0 += kIn) {
+      float2 v[kIn];
+      float4 p[kIn];
+      float mb = M;
+#pragma unroll
+      for (uint32_t k = 0; k < kIn; k++) {
+        const uint32_t c = min(c0 + k, a.nchunk - 1);
+        v[k] = ml[(size_t)c * rows];
+        p[k] = po4[(size_t)c * rows * q4];
+        if (c0 + k >= a.nchunk) v[k].x = -INFINITY;
+        serial |= v[k].x != v[k].x;
+        mb = fmaxf(mb, v[k].x);
+      }
+      if (mb > M) {
+        const float f = __builtin_amdgcn_exp2f(M - mb);
+        L *= f;
+        o = make_float4(o.x * f, o.y * f, o.z * f, o.w * f);
+        M = mb;
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < kIn; k++) {
+        if (!(v[k].x > -INFINITY)) continue;  // nothing was written for an empty split
+        const float f = __builtin_amdgcn_exp2f(v[k].x - M);
+        L = fmaf(v[k].y, f, L);
+        o = make_float4(fmaf(p[k].x, f, o.x), fmaf(p[k].y, f, o.y), fmaf(p[k].z, f, o.z), fmaf(p[k].w, f, o.w));
+      }
+    }
+    w = make_float4(o.x / L, o.y / L, o.z / L, o.w / L);
+    serial |= M == -INFINITY;
+    if (serial && x == 0) atomicOr(&marks, 1u << r);
+  }
+  __syncthreads();
+  for (uint32_t left = marks; left; left &= left - 1) {
+    const uint32_t r1 = __builtin_ctz(left), row1 = blockIdx.x * rpb + r1;
+    float4 w1;
+    const bool ok = attn_row(a, row1 / a.n_heads, row1 % a.n_heads, sc, po, w1);
+    __syncthreads();
+    if (ok) {
+      if (threadIdx.x < q4) po[threadIdx.x] = w1;
+      __syncthreads();
+      if (r == r1) {
+        w = po[x];
+        serial = false;
+      }
+      __syncthreads();
+    }
+  }
+  if (!mine) return;
+  if (serial) w = attn_uniform4(a, row / a.n_heads, row % a.n_heads, 4 * x);
   reinterpret_cast<float4*>(a.ctx)[(size_t)row * q4 + x] = w;
 }
 
@@ -921,8 +1011,8 @@ hipError_t launch_attention_tiled(const AttnArgs& a, hipStream_t st) {
     case 3: hipLaunchKernelGGL(k_attn_tile<3>, grid, dim3(512), 0, st, a); break;
     default: hipLaunchKernelGGL(k_attn_tile<4>, grid, dim3(512), 0, st, a); break;
   }
-  const uint64_t items = (uint64_t)a.n * a.n_heads * (a.hd / 4);
-  hipLaunchKernelGGL(k_attn_merge, dim3((uint32_t)((items + 255) / 256)), dim3(256), 0, st, a);
+  const uint32_t rpb = 256 / (a.hd / 4);
+  hipLaunchKernelGGL(k_attn_merge, dim3((a.n * a.n_heads + rpb - 1) / rpb), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

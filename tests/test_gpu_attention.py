@@ -290,6 +290,27 @@ def test_prompt_tiles_with_non_finite_rows(dev, what):
     assert np.allclose(got[ok], want[ok], rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,bs,window", [(6, 2, 96, 8, 0), (8, 1, 128, 16, 90), (16, 1, 32, 4, 0)])
+def test_prompt_tiles_with_non_finite_rows_over_a_long_span(dev, nh, nkv, hd, bs, window):
+    # several chunks of positions a row, non-finite rows in the cache and in the call, -inf scores
+    # beside finite ones, and every score -inf: as the single-token kernels
+    rng = np.random.default_rng(hd)
+    n = 300
+    q, k, v = (rng.normal(size=(n, w)).astype(np.float32) for w in (nh * hd, nkv * hd, nkv * hd))
+    k[60, 5] = np.inf     # scores of either sign
+    v[150, 7] = np.nan
+    q[200:210] = 0.0      # rows of equal scores: NaN where the infinite key is seen
+    q[230, :] = np.inf
+    kw = dict(block_size=bs, max_positions=400, sliding_window=window, max_seqs=1, rope_theta=1.0)
+    say(f"tiles with non-finite rows hd={hd} window={window}")
+    with KvCache(dev, 1, nh, nkv, hd, **kw) as A, KvCache(dev, 1, nh, nkv, hd, **kw) as B:
+        got = _prompt_calls(A, [A.open_seq()], [n], q, k, v, per=100)
+        want = _prompt_calls(B, [B.open_seq()], [n], q, k, v, per=16)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    assert ok.any() and np.allclose(got[ok], want[ok], rtol=RTOL, atol=ATOL)
+
+
 @pytest.mark.parametrize("nh,nkv,hd,bs,window,bad", [
     (8, 2, 32, 16, 0, None), (32, 8, 128, 16, 70, None), (2, 2, 4, 8, 0, None), (16, 1, 256, 16, 0, None),
     (8, 2, 96, 16, 64, None), (32, 8, 128, 16, 0, "nan"), (8, 2, 32, 5, 0, "inf")])
