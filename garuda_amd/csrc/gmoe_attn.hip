@@ -111,9 +111,10 @@ __global__ void __launch_bounds__(256) k_rope_rows(AttnArgs a) {
   if (t == 0 && blockIdx.y == 0) {
     const_cast<AttnEntry*>(a.ent)[i] = e;
     if (i < a.ntile) const_cast<AttnTile*>(a.tiles)[i] = a.htile[i];
+    if (i < a.npick) const_cast<uint32_t*>(a.pick)[i] = a.hpick[i];
   }
   const uint32_t slot = e.pos % a.bs, kvd = a.n_kv * a.hd, nh = a.n_heads + a.n_kv, step = ng * gridDim.y;
-  if (e.fresh && t == 0 && blockIdx.y == 0) e.pages[e.pos / a.bs] = e.page;  // read by the attention kernel after this one
+  if ((e.fresh & 1) && t == 0 && blockIdx.y == 0) e.pages[e.pos / a.bs] = e.page;  // read by the attention kernel after this one
   float* kp = a.pool + (size_t)e.page * a.page_floats + (size_t)slot * a.hd;  // head h at + h * bs * hd
   float* vp = kp + (size_t)a.bs * kvd;
   const float* vs = a.v + (size_t)i * a.kv_stride;
@@ -181,7 +182,7 @@ __global__ void __launch_bounds__(256) k_attn_partial(AttnArgs a) {
   constexpr int NR = MAXHD / 16;  // float4 columns of a row per thread
   extern __shared__ float4 lds_v4[];
   float* lds_f = reinterpret_cast<float*>(lds_v4);
-  const uint32_t i = blockIdx.x, h = blockIdx.y, c = blockIdx.z, t = threadIdx.x;
+  const uint32_t i = !ROPE && a.pick ? a.pick[blockIdx.x] : blockIdx.x, h = blockIdx.y, c = blockIdx.z, t = threadIdx.x;
   const uint32_t G = a.n_heads / a.n_kv, hd = a.hd, kvd = a.n_kv * hd, q4 = hd / 4;
   float* tile = lds_f;                  // [kAttnChunk][hd] values
   float* qs = tile + kAttnChunk * hd;   // [G][hd]
@@ -192,7 +193,7 @@ __global__ void __launch_bounds__(256) k_attn_partial(AttnArgs a) {
   auto ml = [&](uint32_t g, uint32_t k) -> float& { return mlb[2 * g + k]; };
   const AttnEntry e = entry(a, i);
   const uint32_t end = e.pos + 1, p0 = e.start + c * kAttnChunk;
-  float* out = a.part + (((size_t)i * a.n_heads + h * G) * a.nchunk + c) * (hd + 2);
+  float* out = a.part + (((size_t)blockIdx.x * a.n_heads + h * G) * a.nchunk + c) * (hd + 2);
   const size_t gstride = (size_t)a.nchunk * (hd + 2);
   if (p0 >= end) {  // past the entry's span: an empty chunk
     if (t < G) {
@@ -412,8 +413,8 @@ __device__ float attn_uniform(const AttnArgs& a, uint32_t i, uint32_t hh, uint32
 // +inf score), or no finite score at all, gives the uniform weights of attn_uniform.
 __global__ void __launch_bounds__(256) k_attn_combine(AttnArgs a) {
   __shared__ float gm[256], gl[256], go[256];
-  const uint32_t i = blockIdx.x, hh = blockIdx.y, t = threadIdx.x, hd = a.hd, row = hd + 2, nc = a.nchunk;
-  const float* base = a.part + ((size_t)i * a.n_heads + hh) * nc * row;
+  const uint32_t i = a.pick ? a.pick[blockIdx.x] : blockIdx.x, hh = blockIdx.y, t = threadIdx.x, hd = a.hd, row = hd + 2, nc = a.nchunk;
+  const float* base = a.part + ((size_t)blockIdx.x * a.n_heads + hh) * nc * row;
   const uint32_t ng = 256 / hd, g = t / hd, d = t % hd;
   float M = -INFINITY, L = 0.0f, O = 0.0f;
   bool bad = false;
@@ -896,7 +897,7 @@ __global__ void __launch_bounds__(256) k_attn_merge(AttnArgs a) {
   __shared__ uint32_t marks;
   const uint32_t rows = a.n * a.n_heads, q4 = a.hd / 4, rpb = 256 / q4, r = threadIdx.x / q4, x = threadIdx.x % q4;
   const uint32_t row = blockIdx.x * rpb + r;
-  const bool mine = r < rpb && row < rows;
+  const bool mine = r < rpb && row < rows && !(a.npick && (a.ent[row / a.n_heads].fresh & kAttnSingle));
   float4 w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   bool serial = false;
   if (threadIdx.x == 0) marks = 0;
@@ -967,7 +968,7 @@ static void launch_partial(const AttnArgs& a, hipStream_t st) {
       hipFuncSetAttribute((const void*)k_attn_partial<kAttnMaxHd, ROPE, ONE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)attn_lds_bytes(kAttnMaxGroup, kAttnMaxHd)) == hipSuccess;
   (void)once;
-  const dim3 grid(a.n, a.n_kv, a.nchunk);
+  const dim3 grid(a.pick ? a.npick : a.n, a.n_kv, a.nchunk);
   const uint32_t lds = attn_lds_bytes(a.n_heads / a.n_kv, a.hd);
   if (a.hd <= 128) hipLaunchKernelGGL((k_attn_partial<128, ROPE, ONE>), grid, dim3(256), lds, st, a);
   else hipLaunchKernelGGL((k_attn_partial<kAttnMaxHd, ROPE, ONE>), grid, dim3(256), lds, st, a);
@@ -1002,8 +1003,8 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_attention_tiled(const AttnArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL(k_rope_rows, dim3(a.n, 2), dim3(256), 0, st, a);
+hipError_t launch_attention_tiled(const AttnArgs& a, const AttnArgs& rest, hipStream_t st) {
+  hipLaunchKernelGGL(k_rope_rows, dim3(a.n, 2), dim3(256), 0, st, a);  // every entry's k and v before any attends
   const dim3 grid(a.n_kv, a.ntile, a.nchunk);
   switch (a.hd / 32) {
     case 1: hipLaunchKernelGGL(k_attn_tile<1>, grid, dim3(512), 0, st, a); break;
@@ -1013,6 +1014,10 @@ hipError_t launch_attention_tiled(const AttnArgs& a, hipStream_t st) {
   }
   const uint32_t rpb = 256 / (a.hd / 4);
   hipLaunchKernelGGL(k_attn_merge, dim3((a.n * a.n_heads + rpb - 1) / rpb), dim3(256), 0, st, a);
+  if (a.npick) {
+    launch_partial<false, false>(rest, st);
+    hipLaunchKernelGGL(k_attn_combine, dim3(a.npick, a.n_heads), dim3(256), 0, st, rest);
+  }
   return hipGetLastError();
 }
 

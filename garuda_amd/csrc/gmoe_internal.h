@@ -418,8 +418,10 @@ struct AttnEntry {
   uint32_t pos;     // this token's position
   uint32_t start;   // first position it attends to (sliding window)
   uint32_t page;    // the page holding pos
-  uint32_t fresh;   // 1: pos opens that page; the append records it in the table
+  uint32_t fresh;   // 1: pos opens that page; the append records it in the table. In a tiled
+                    // call also kAttnSingle: the entry is in no tile
 };
+constexpr uint32_t kAttnSingle = 2;
 
 // Rows r0 .. r0 + nr - 1 of a run: consecutive entries of one sequence from entry i0 on,
 // row r being token r / G's query head r % G of a kv head's group of G.
@@ -449,7 +451,10 @@ struct AttnArgs {
   uint32_t nchunk;       // chunks of kAttnChunk positions per entry (tiled: splits of skeys)
   const AttnTile* tiles; // tiled calls (launch_attention_tiled): [ntile], and the keys of a split;
   const AttnEntry* hent; //   their entries and tiles in pinned host memory, which the first launch
-  const AttnTile* htile; //   copies to ent and tiles (a copy of its own cost 9.5 us a call)
+  const AttnTile* htile; //   copies to ent and tiles (a copy of its own cost 9.5 us a call), and
+  const uint32_t* hpick; //   the npick entries that are in no tile (kAttnSingle), copied to pick
+  const uint32_t* pick;  // single-token kernels: entry pick[x] for workgroup x, or null: entry x
+  uint32_t npick;
   uint32_t ntile, skeys; //   part is then [nchunk][n * n_heads][hd] o, then [nchunk][n * n_heads][2] (m, l)
   float* ctx;            // [n][n_heads * hd]
   uint32_t q_stride, kv_stride;  // floats between consecutive rows of q, and of k and v
@@ -459,8 +464,9 @@ struct AttnArgs {
 
 constexpr uint32_t kAttnChunk = 64, kAttnMaxGroup = 16, kAttnMaxHd = 256;
 hipError_t launch_attention(const AttnArgs& a, hipStream_t st);
-// Runs of several tokens of one sequence (prompts): attn_tiled_hd says which head widths.
-hipError_t launch_attention_tiled(const AttnArgs& a, hipStream_t st);
+// Runs of several tokens of one sequence (prompts): attn_tiled_hd says which head widths. rest
+// (a's with its own part and nchunk) attends a.npick entries by the single-token kernels.
+hipError_t launch_attention_tiled(const AttnArgs& a, const AttnArgs& rest, hipStream_t st);
 constexpr bool attn_tiled_hd(uint32_t hd) { return hd % 32 == 0 && hd <= 128; }
 
 // Decode-step glue (gmoe_glue.hip): embedding rows, residual add + RMSNorm * weight,

@@ -6,7 +6,7 @@
 // blocks are pages of one device pool shared by every sequence and layer; the host keeps
 // each (sequence, layer)'s length and page list, and the device keeps its page table,
 // which the append kernel extends when a token opens a page. attend_one
-// (llama/mod.rs:766-821) runs as three launches (gmoe_attn.hip).
+// (llama/mod.rs:766-821) runs as one to five launches (gmoe_attn.hip).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -48,7 +48,8 @@ gmoe_status kfail(gmoe_status s, const char* fmt, ...) {
   } while (0)
 
 constexpr size_t kPinHalf = (size_t)512 << 10;  // bytes of a half at least
-constexpr size_t kPinEntry = sizeof(AttnEntry) + sizeof(AttnTile);  // a call has at most one tile per entry
+// a call has at most one tile per entry, and a place in the list of those in none
+constexpr size_t kPinEntry = sizeof(AttnEntry) + sizeof(AttnTile) + sizeof(uint32_t);
 
 struct Seq {
   bool open = false;
@@ -108,8 +109,10 @@ gmoe_status grow_scratch(gmoe_kv* kv, size_t bytes) {
 gmoe_status take_pinned(gmoe_kv* kv, size_t bytes, hipStream_t st, uint8_t** out) {
   bytes = (bytes + 63) & ~(size_t)63;
   if (bytes > kv->pin_half) {
-    KV_TRY(hipDeviceSynchronize());  // queued calls may still read the old buffer
-    if (kv->pin) KV_TRY(hipHostFree(kv->pin));
+    if (kv->pin) {
+      KV_TRY(hipDeviceSynchronize());  // queued calls may still read the old buffer
+      KV_TRY(hipHostFree(kv->pin));
+    }
     kv->pin = nullptr;
     kv->pin_half = kv->pin_at = 0;
     const size_t half = std::max(bytes, kPinHalf);
@@ -128,17 +131,21 @@ gmoe_status take_pinned(gmoe_kv* kv, size_t bytes, hipStream_t st, uint8_t** out
 }
 
 // The call's entries (positions, windows, pages), checked against the window and the
-// free pages but not committed; maxspan receives the longest span attended.
-gmoe_status plan(gmoe_kv* kv, uint32_t layer, const uint32_t* seqs, uint32_t n, AttnEntry* ent, uint32_t* maxspan) {
+// free pages but not committed; maxspan receives the longest span attended, distinct whether
+// no two entries are of one sequence.
+gmoe_status plan(gmoe_kv* kv, uint32_t layer, const uint32_t* seqs, uint32_t n, AttnEntry* ent, uint32_t* maxspan,
+                 bool* distinct = nullptr) {
   const gmoe_kv_desc& D = kv->d;
   if (layer >= D.n_layers) return kfail(GMOE_ERR_INFERENCE, "layer %u of %u", layer, D.n_layers);
   if (n == 0 || !seqs) return kfail(GMOE_ERR_INFERENCE, "empty attention call");
   std::vector<uint32_t> extra(kv->seqs.size(), 0);  // this call's entries so far, per sequence
   uint32_t need_pages = 0;
   *maxspan = 1;
+  bool once = true;
   for (uint32_t i = 0; i < n; i++) {
     const uint32_t s = seqs[i];
     if (s >= kv->seqs.size() || !kv->seqs[s].open) return kfail(GMOE_ERR_INFERENCE, "sequence %u is not open", s);
+    once &= extra[s] == 0;
     const uint32_t pos = kv->seqs[s].len[layer] + extra[s]++;
     if (pos >= D.max_positions)
       return kfail(GMOE_ERR_CACHE, "context window of %u positions is exhausted", D.max_positions);
@@ -152,6 +159,7 @@ gmoe_status plan(gmoe_kv* kv, uint32_t layer, const uint32_t* seqs, uint32_t n, 
   if (need_pages > kv->free_pages.size())
     return kfail(GMOE_ERR_CACHE, "the KV pool has %zu free pages, the call needs %u", kv->free_pages.size(),
                  need_pages);
+  if (distinct) *distinct = once;
   return GMOE_OK;
 }
 
@@ -173,27 +181,62 @@ void commit(gmoe_kv* kv, uint32_t layer, const uint32_t* seqs, uint32_t n, AttnE
   }
 }
 
-// A call above kAttnInline tokens whose entries come in runs (consecutive entries of one
-// sequence: a prompt's positions) is cut into tiles of kAttnTileRows (token, query head)
-// rows. Runs shorter than an eighth of a tile on average leave the MFMA rows mostly empty and
-// take the kernels of single tokens (no tiles), as do decode batches. span receives the most keys a tile reads.
-std::vector<AttnTile> tile_runs(const gmoe_kv* kv, const AttnEntry* ent, uint32_t n, uint32_t* span) {
-  const uint32_t G = kv->d.n_heads / kv->d.n_kv_heads;
+// Workgroups a tiled call is split into at least, keys permitting: a tile's keys are split over
+// workgroups until the call has about one workgroup a CU, each split keeping at least two key
+// tiles. The key tiles of a split:
+constexpr uint32_t kAttnTileWgs = 256;
+uint32_t split_key_tiles(const gmoe_kv* kv, size_t ntile, uint32_t span) {
+  const uint32_t kt = (span + kAttnTileKeys - 1) / kAttnTileKeys;
+  const uint32_t wgs = (uint32_t)ntile * kv->d.n_kv_heads;
+  const uint32_t ns = std::max(1u, std::min((kAttnTileWgs + wgs - 1) / wgs, kt / 2));
+  return (kt + ns - 1) / ns;
+}
+
+// How a call's entries are attended. Above kAttnInline tokens, runs (consecutive entries of one
+// sequence: a prompt's positions) of at least an eighth of a tile of rows are cut into tiles of
+// kAttnTileRows (token, query head) rows. Shorter runs leave the MFMA rows mostly empty: decode
+// batches have no tiles, and beside a prompt such runs are singles, attended token by token in
+// two more launches, unless as tiles of their own they leave every split with few keys. 32 heads
+// on 8 of 128, 300 prompt tokens beside 30 sequences at 4000: all in tiles 630 us, singles apart
+// 350, all token by token 874; 8 heads on 2 of 32, 64 tokens beside 3 sequences at 3000: 23, 33 and 30.
+// span and chunks: the most keys a tile reads, and the most chunks of kAttnChunk a single attends.
+struct Runs {
   std::vector<AttnTile> tiles;
-  *span = 1;
-  if (n <= kAttnInline || !attn_tiled_hd(kv->d.head_dim)) return tiles;
-  for (uint32_t i = 0, j; i < n; i = j) {
-    for (j = i + 1; j < n && ent[j].pages == ent[i].pages;) j++;
-    const uint32_t rows = (j - i) * G;
-    for (uint32_t r = 0; r < rows; r += kAttnTileRows) {
-      const uint32_t nr = std::min(kAttnTileRows, rows - r);
-      const AttnEntry &f = ent[i + r / G], &e = ent[i + (r + nr - 1) / G];
-      *span = std::max(*span, e.pos + 1 - f.start);
-      tiles.push_back(AttnTile{i, r, nr, f.start, f.pos, e.start, e.pos, 0, f.pages});
+  std::vector<uint32_t> singles;
+  uint32_t span = 1, chunks = 1;
+};
+constexpr uint32_t kAttnFewKeyTiles = 4;
+Runs find_runs(const gmoe_kv* kv, const AttnEntry* ent, uint32_t n, const float* out) {
+  const uint32_t G = kv->d.n_heads / kv->d.n_kv_heads;
+  // the tiles' rows are written 16 bytes at a time
+  if (n <= kAttnInline || !attn_tiled_hd(kv->d.head_dim) || (uintptr_t)out % 16) return {};
+  auto find = [&](bool short_too) {
+    Runs R;
+    for (uint32_t i = 0, j; i < n; i = j) {
+      for (j = i + 1; j < n && ent[j].pages == ent[i].pages;) j++;
+      const uint32_t rows = (j - i) * G;
+      if (!short_too && 8 * rows < kAttnTileRows) {
+        for (uint32_t k = i; k < j; k++) {
+          R.singles.push_back(k);
+          R.chunks = std::max(R.chunks, (ent[k].pos - ent[k].start) / kAttnChunk + 1);
+        }
+        continue;
+      }
+      for (uint32_t r = 0; r < rows; r += kAttnTileRows) {
+        const uint32_t nr = std::min(kAttnTileRows, rows - r);
+        const AttnEntry &f = ent[i + r / G], &e = ent[i + (r + nr - 1) / G];
+        R.span = std::max(R.span, e.pos + 1 - f.start);
+        R.tiles.push_back(AttnTile{i, r, nr, f.start, f.pos, e.start, e.pos, 0, f.pages});
+      }
     }
-  }
-  if ((uint64_t)n * G * 8 < (uint64_t)tiles.size() * kAttnTileRows) tiles.clear();
-  return tiles;
+    return R;
+  };
+  Runs R = find(false);
+  if (R.singles.empty()) return R;
+  // few tokens in tiles beside others are not worth two more launches
+  if (n - R.singles.size() <= kAttnInline) return {};
+  Runs all = find(true);
+  return split_key_tiles(kv, all.tiles.size(), all.span) <= kAttnFewKeyTiles ? all : R;
 }
 
 // Scratch of a call of n entries and nchunk chunks: entries and tiles, rotated q, partials.
@@ -236,59 +279,61 @@ AttnArgs args(const gmoe_kv* kv, uint32_t n, uint32_t nchunk, const AttnLayout& 
   return a;
 }
 
-// Workgroups a tiled call is split into at least, keys permitting.
-constexpr uint32_t kAttnTileWgs = 256;
-
 // Plans the call's entries and commits them (lengths advance and pages are taken only when
 // the whole call fits), then queues the launches.
 gmoe_status attend(gmoe_kv* kv, uint32_t layer, const uint32_t* seqs, uint32_t n, const float* q, const float* k,
                    const float* v, float* out, hipStream_t st, uint32_t q_stride = 0, uint32_t kv_stride = 0) {
   std::vector<AttnEntry> ent(n ? n : 1);
   uint32_t maxspan;
-  if (gmoe_status s = plan(kv, layer, seqs, n, ent.data(), &maxspan)) return s;
-  uint32_t span;
-  std::vector<AttnTile> tiles = tile_runs(kv, ent.data(), n, &span);
-  if ((uintptr_t)out % 16) tiles.clear();  // its rows are written 16 bytes at a time
+  bool distinct;
+  if (gmoe_status s = plan(kv, layer, seqs, n, ent.data(), &maxspan, &distinct)) return s;
+  const Runs R = find_runs(kv, ent.data(), n, out);
+  const uint32_t ntile = (uint32_t)R.tiles.size(), npick = ntile ? (uint32_t)R.singles.size() : 0;
   uint32_t nchunk = (maxspan + kAttnChunk - 1) / kAttnChunk, skeys = 0;
-  if (!tiles.empty()) {
-    // a tile's keys split over workgroups until the call has about one workgroup a CU,
-    // each split keeping at least two key tiles
-    const uint32_t kt = (span + kAttnTileKeys - 1) / kAttnTileKeys;
-    const uint32_t wgs = (uint32_t)tiles.size() * kv->d.n_kv_heads;
-    const uint32_t ns = std::max(1u, std::min((kAttnTileWgs + wgs - 1) / wgs, kt / 2));
-    skeys = (kt + ns - 1) / ns * kAttnTileKeys;
-    nchunk = (span + skeys - 1) / skeys;
+  if (ntile) {
+    skeys = split_key_tiles(kv, ntile, R.span) * kAttnTileKeys;
+    nchunk = (R.span + skeys - 1) / skeys;
   }
-  const AttnLayout l = layout(kv, n, nchunk);
+  AttnLayout l = layout(kv, n, nchunk);
+  const size_t o_rest = (l.total + 255) & ~(size_t)255;  // the singles' partials
+  if (npick) l.total = o_rest + (size_t)npick * kv->d.n_heads * R.chunks * (kv->d.head_dim + 2) * 4;
   if (gmoe_status s = grow_scratch(kv, l.total)) return s;
-  const size_t eb = n * sizeof(AttnEntry), tb = tiles.size() * sizeof(AttnTile);
+  const size_t eb = n * sizeof(AttnEntry), tb = ntile * sizeof(AttnTile), pb = npick * sizeof(uint32_t);
   uint8_t* pin = nullptr;
   if (n > kAttnInline)
-    if (gmoe_status s = take_pinned(kv, eb + tb, st, &pin)) return s;
+    if (gmoe_status s = take_pinned(kv, eb + tb + pb, st, &pin)) return s;
   commit(kv, layer, seqs, n, ent.data());
+  for (uint32_t i = 0; i < npick; i++) ent[R.singles[i]].fresh |= kAttnSingle;
   AttnArgs a = args(kv, n, nchunk, l, q, k, v, out, q_stride, kv_stride);
   if (n <= kAttnInline) {  // a decode batch: the entries ride in the kernel arguments
     std::copy(ent.begin(), ent.begin() + n, a.inl);
     a.ent = nullptr;
-    a.distinct = 1;
-    for (uint32_t i = 0; i < n; i++)
-      for (uint32_t j = 0; j < i; j++)
-        if (ent[j].pages == ent[i].pages) a.distinct = 0;
   } else {
     memcpy(pin, ent.data(), eb);
-    if (tb) memcpy(pin + eb, tiles.data(), tb);
-    a.ent = reinterpret_cast<const AttnEntry*>(kv->scratch + l.o_ent);
-    if (tb) {
-      a.tiles = reinterpret_cast<const AttnTile*>(kv->scratch + l.o_ent + eb);
+    uint8_t* dev = kv->scratch + l.o_ent;
+    a.ent = reinterpret_cast<const AttnEntry*>(dev);
+    if (ntile) {
+      memcpy(pin + eb, R.tiles.data(), tb);
+      if (pb) memcpy(pin + eb + tb, R.singles.data(), pb);
+      a.tiles = reinterpret_cast<const AttnTile*>(dev + eb);
       a.hent = reinterpret_cast<const AttnEntry*>(pin);
       a.htile = reinterpret_cast<const AttnTile*>(pin + eb);
-      a.ntile = (uint32_t)tiles.size();
+      a.ntile = ntile;
       a.skeys = skeys;
-      KV_TRY(launch_attention_tiled(a, st));
+      if (npick) {
+        a.pick = reinterpret_cast<const uint32_t*>(dev + eb + tb);
+        a.hpick = reinterpret_cast<const uint32_t*>(pin + eb + tb);
+        a.npick = npick;
+      }
+      AttnArgs rest = a;
+      rest.part = reinterpret_cast<float*>(kv->scratch + o_rest);
+      rest.nchunk = R.chunks;
+      KV_TRY(launch_attention_tiled(a, rest, st));
       return GMOE_OK;
     }
-    KV_TRY(hipMemcpyAsync(kv->scratch + l.o_ent, pin, eb, hipMemcpyHostToDevice, st));
+    KV_TRY(hipMemcpyAsync(dev, pin, eb, hipMemcpyHostToDevice, st));
   }
+  a.distinct = distinct ? 1 : 0;
   KV_TRY(launch_attention(a, st));
   return GMOE_OK;
 }

@@ -311,6 +311,58 @@ def test_prompt_tiles_with_non_finite_rows_over_a_long_span(dev, nh, nkv, hd, bs
     assert ok.any() and np.allclose(got[ok], want[ok], rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,bs,window,order,tokens", [
+    (32, 8, 128, 16, 0, "pssps", (40, 1)), (8, 8, 64, 16, 0, "sspss", (33, 2)),  # group 1: runs from 32 tokens tile
+    (16, 1, 32, 4, 70, "spspspss", (20, 1)), (8, 2, 96, 5, 0, "ssssssssssssssssssssp", (90, 1)),
+    (8, 2, 64, 16, 0, "pssss", (9, 3)),  # nine tokens of four rows fill an eighth of a tile, too few to tile beside others
+    (8, 2, 64, 16, 0, "pspss", (9, 7)), (64, 64, 32, 16, 0, "pssss", (40, 1))])
+def test_prompts_beside_decoding_sequences(dev, nh, nkv, hd, bs, window, order, tokens):
+    # One call of prompts (p) and decoding sequences (s) at their own lengths: the prompts' rows in
+    # tiles, the others in tiles too or, where those would have many keys, token by token (64 kv
+    # heads). Each sequence by itself in calls of at most 16 tokens: within the layer tolerance, and
+    # the same bits token by token.
+    rng = np.random.default_rng(len(order) + hd)
+    w = (nh * hd, nkv * hd, nkv * hd)
+    kw = dict(block_size=bs, max_positions=400, sliding_window=window, max_seqs=len(order))
+    say(f"mixed call hd={hd} {order}")
+    with KvCache(dev, 1, nh, nkv, hd, **kw) as A, KvCache(dev, 1, nh, nkv, hd, **kw) as B:
+        ids, runs, at = [], [], 0
+        for s, c in enumerate(order):
+            assert A.open_seq() == B.open_seq() == s
+            past = int(rng.integers(1, 200))
+            x = [rng.normal(size=(past, y)).astype(np.float32) for y in w]
+            for kv in (A, B):
+                _prompt_calls(kv, [s], [past], *x, per=16)
+            m = tokens["ps".index(c)]
+            ids += [s] * m
+            runs.append((s, c, slice(at, at + m)))
+            at += m
+        for turn in range(2):
+            q, k, v = (rng.normal(size=(at, y)).astype(np.float32) for y in w)
+            got = A.attention(0, ids, q, k, v)
+            for s, c, r in runs:
+                want = _prompt_calls(B, [s], [r.stop - r.start], q[r], k[r], v[r], per=16)
+                if c == "s" and nkv == 64:
+                    assert np.array_equal(bits(got[r]), bits(want)), f"sequence {s}"
+                check(got[r], want, f"sequence {s}")
+
+
+def test_large_decode_batch_is_the_same_bits_as_small_ones(dev):
+    # above 16 sequences the entries go through device memory; each sequence's rotation and
+    # append still ride in the attention's own launch
+    nh, nkv, hd, n = 8, 2, 64, 37
+    rng = np.random.default_rng(3)
+    with KvCache(dev, 1, nh, nkv, hd, max_seqs=n) as A, KvCache(dev, 1, nh, nkv, hd, max_seqs=n) as B:
+        a, b = [A.open_seq() for _ in range(n)], [B.open_seq() for _ in range(n)]
+        for step in range(70):
+            m = n - step % 3
+            q, k, v = (rng.normal(size=(m, w)).astype(np.float32) for w in (nh * hd, nkv * hd, nkv * hd))
+            got = A.attention(0, a[:m], q, k, v)
+            want = np.concatenate([B.attention(0, b[i:min(i + 16, m)], q[i:i + 16], k[i:i + 16], v[i:i + 16])
+                                   for i in range(0, m, 16)])
+            assert np.array_equal(bits(got), bits(want)), f"step {step}"
+
+
 @pytest.mark.parametrize("nh,nkv,hd,bs,window,bad", [
     (8, 2, 32, 16, 0, None), (32, 8, 128, 16, 70, None), (2, 2, 4, 8, 0, None), (16, 1, 256, 16, 0, None),
     (8, 2, 96, 16, 64, None), (32, 8, 128, 16, 0, "nan"), (8, 2, 32, 5, 0, "inf")])
