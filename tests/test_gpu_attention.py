@@ -388,6 +388,53 @@ def test_decode_launch_with_rotation_is_the_same_bits(dev, nh, nkv, hd, bs, wind
             assert same.all(), f"step {step}: {np.count_nonzero(~same)} differ"
 
 
+def test_pinned_entries_survive_until_their_call_has_run(dev):
+    # Calls above 16 tokens put their entries (24 bytes) and tiles into two pinned halves of 512 KiB,
+    # 35 calls of 600 tokens each: 150 calls queued without a wait go round both twice, then one of
+    # 22000 tokens needs a larger buffer while calls are queued, and more follow. A cache whose
+    # stream is waited for after every call gives the same contexts.
+    import ctypes as C
+    hip = _hip()
+    nh, nkv, hd, n, big = 2, 1, 32, 600, 22000
+    rng = np.random.default_rng(8)
+    x = [rng.normal(size=(big, w * hd)).astype(np.float32) for w in (nh, nkv, nkv)]
+    calls = [(i % 3, n) for i in range(150)] + [(3, big)] + [(i % 3, n) for i in range(4)]
+    bufs = []
+
+    def device(nbytes, src=None):
+        b = C.c_void_p()
+        assert hip.hipMalloc(C.byref(b), nbytes) == 0
+        bufs.append(b)
+        if src is not None:
+            assert hip.hipMemcpy(b, src.ctypes.data, nbytes, 1) == 0
+        return b.value
+
+    kw = dict(block_size=16, max_positions=32000, sliding_window=100, max_seqs=4)
+    try:
+        d = [device(t.nbytes, t) for t in x]
+        out = []
+        say("pinned ring")
+        for wait in (False, True):
+            with KvCache(dev, 1, nh, nkv, hd, **kw) as kv:
+                ids = [kv.open_seq() for _ in range(4)]
+                o = device(4 * nh * hd * sum(m for _, m in calls))
+                at, res = 0, np.empty((sum(m for _, m in calls), nh * hd), np.float32)
+                for i, (s, m) in enumerate(calls):
+                    r = 0 if m == big else 7 * i  # other rows every call
+                    q, k, v = (b + 4 * r * t.shape[1] for b, t in zip(d, x))
+                    kv.attention_async(0, [ids[s]] * m, q, k, v, o + 4 * nh * hd * at, 0)
+                    at += m
+                    if wait:
+                        assert hip.hipDeviceSynchronize() == 0
+                assert hip.hipDeviceSynchronize() == 0
+                assert hip.hipMemcpy(res.ctypes.data, o, res.nbytes, 2) == 0
+                out.append(res)
+        assert np.isfinite(out[0]).all() and np.array_equal(bits(out[0]), bits(out[1]))
+    finally:
+        for b in bufs:
+            hip.hipFree(b)
+
+
 def test_decode_context_over_its_query(dev):
     # the context may lie over the call's q, as when a caller reuses the buffer
     import ctypes as C
