@@ -411,9 +411,11 @@ __device__ float attn_uniform(const AttnArgs& a, uint32_t i, uint32_t hh, uint32
 // d (16 chunks in flight) with a running max: (M, L, O) is rescaled when a chunk's max
 // exceeds M. The groups are then merged in group order. A chunk marked NaN (a NaN or
 // +inf score), or no finite score at all, gives the uniform weights of attn_uniform.
+// PICK: the entries of a.pick.
+template <bool PICK>
 __global__ void __launch_bounds__(256) k_attn_combine(AttnArgs a) {
   __shared__ float gm[256], gl[256], go[256];
-  const uint32_t i = a.pick ? a.pick[blockIdx.x] : blockIdx.x, hh = blockIdx.y, t = threadIdx.x, hd = a.hd, row = hd + 2, nc = a.nchunk;
+  const uint32_t i = PICK ? a.pick[blockIdx.x] : blockIdx.x, hh = blockIdx.y, t = threadIdx.x, hd = a.hd, row = hd + 2, nc = a.nchunk;
   const float* base = a.part + ((size_t)blockIdx.x * a.n_heads + hh) * nc * row;
   const uint32_t ng = 256 / hd, g = t / hd, d = t % hd;
   float M = -INFINITY, L = 0.0f, O = 0.0f;
@@ -999,7 +1001,7 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(k_rope_append, dim3(a.n, (pairs + 255) / 256), dim3(256), 0, st, a);
     launch_partial<false, false>(a, st);
   }
-  hipLaunchKernelGGL(k_attn_combine, dim3(a.n, a.n_heads), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(k_attn_combine<false>, dim3(a.n, a.n_heads), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
@@ -1016,7 +1018,7 @@ hipError_t launch_attention_tiled(const AttnArgs& a, const AttnArgs& rest, hipSt
   hipLaunchKernelGGL(k_attn_merge, dim3((a.n * a.n_heads + rpb - 1) / rpb), dim3(256), 0, st, a);
   if (a.npick) {
     launch_partial<false, false>(rest, st);
-    hipLaunchKernelGGL(k_attn_combine, dim3(a.npick, a.n_heads), dim3(256), 0, st, rest);
+    hipLaunchKernelGGL(k_attn_combine<true>, dim3(a.npick, a.n_heads), dim3(256), 0, st, rest);
   }
   return hipGetLastError();
 }
