@@ -1621,15 +1621,15 @@ hipError_t launch_pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hip
 // the tokens, by a step after every 8, and with the rows; k_pq's hardly does up to 32 tokens,
 // and is least for the types of 32-value sub-blocks. Both give a row the same bits, so the
 // line is one of time only. Decode kernels and k_pq, us, columns 4096:
-//   rows 4096:  Q4_K 17 tokens 22.2 and 21.0, Q5_K 22.4 and 22.8, Q8_0 23.8 and 21.5, Q2_K 29.1
-//               and 28.0; Q3_K 24 tokens 26.5 and 26.0, Q6_K 24 tokens 27.5 and 29.7, 32 35.3 and 33.9;
+//   rows 4096:  Q4_K 17 tokens 22.2 and 21.0, Q5_K 22.4 and 22.8 (20 tokens 23.4 and 23.2), Q8_0 23.8 and
+//               21.5, Q2_K 29.1 and 28.0; Q3_K 24 tokens 26.5 and 26.0, Q6_K 24 tokens 27.5 and 29.7, 32 35.3 and 33.9;
 //   rows 14336: 17 tokens Q4_K 62.7 and 34.1, Q3_K 64.7 and 45.3, Q6_K 79.2 and 80.0 (20 tokens 96.3
 //               and 80.3); rows 32000: Q6_K 17 tokens 96.4 and 87.4, 64 tokens 313 and 164;
 //   rows 1024:  Q4_K 24 tokens 21.1 and 21.5, 32 27.6 and 23.3; Q3_K 32 tokens 29.4 and 30.0, 40
 //               32.7 and 31.1; Q6_K 40 tokens 34.3 and 35.2.
 static uint32_t pq_dense_min(uint32_t qt, uint32_t rows) {
   if (rows < 4096) return qt == Q6_K ? 48 : qt == Q3_K ? 40 : 32;
-  if (rows < 8192) return qt == Q6_K ? 32 : qt == Q3_K ? 24 : 17;
+  if (rows < 8192) return qt == Q6_K ? 32 : qt == Q3_K ? 24 : qt == Q5_K ? 20 : 17;
   return 17;
 }
 
