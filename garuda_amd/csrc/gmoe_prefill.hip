@@ -1237,24 +1237,28 @@ hipError_t pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_
   }
 }
 
-// Tokens of a packed-math dense workgroup, and whether it folds the K slices. 64 tokens (types
-// of 16-value sub-blocks, whose decoding 32 tokens do not pay for: the Q6_K head at 64 tokens
-// 164 us, with 32 a workgroup 198) where the grid then still fills three quarters of the
-// chip; else 32, which fits three workgroups a CU with 32-value sub-blocks. Folded where the
-// tiles alone fill the chip, so that no slices are written (Q4_K, 4096 x 4096 at 2048 tokens
-// 267 us, in slices 289); below, a workgroup a slice (at 250 tokens 47.6, folded 118).
+// Tokens of a packed-math dense workgroup, and whether it folds the K slices. 32 tokens leave
+// registers for three workgroups a CU (two with 16-value sub-blocks) and a time that follows
+// their number; 64 decode a weight half as often, two a CU, in rounds of all places, and are
+// taken where those are nearly full (4096 x 4096, Q4_K: 250 tokens 47.4 us with 32 and 44.0
+// with 64, 320 tokens 52.8 and 65.4; Q3_K 66.3 and 59.8, 81.6 and 91.2). Q6_K holds one
+// workgroup a CU either way and takes 64 from three quarters of a round (the head of 32000 rows
+// at 64 tokens 198 and 164). Folded where the tiles alone fill the chip, so that no slices are
+// written (Q4_K, 4096 x 4096 at 2048 tokens 241 us, in slices 320); below, a workgroup a slice (at
+// 250 tokens folded 118).
 template <int QT>
 PqDense pq_dense_split(const LayerDev& L, uint32_t n, uint32_t ksg) {
   PqDense p{32, false};
   if constexpr (pq_type<QT>()) {
-    const uint32_t row_tiles = L.d / pf_rows<QT>(false), wide = row_tiles * ((n + 63) / 64);
-    uint32_t tiles = row_tiles * ((n + 31) / 32), slots = 256 * pq_waves<QT, false, 32>();
-    if (PQ<QT>::SBW == 16 && n > 32 && 4 * wide * ksg >= 3 * 256 * pq_waves<QT, false, 64>()) {
-      p.tok = 64;
-      tiles = wide;
-      slots = 256 * pq_waves<QT, false, 64>();
-    }
-    p.fold = tiles >= slots;
+    const uint32_t row_tiles = L.d / pf_rows<QT>(false), tiles32 = row_tiles * ((n + 31) / 32);
+    const uint32_t tiles64 = row_tiles * ((n + 63) / 64);
+    const uint32_t slots32 = 256 * pq_waves<QT, false, 32>(), slots64 = 256 * pq_waves<QT, false, 64>();
+    const bool fold64 = tiles64 >= slots64, fold32 = tiles32 >= slots32;
+    const uint32_t k64 = fold64 ? 1 : ksg, rounds64 = (tiles64 * k64 + slots64 - 1) / slots64;
+    const bool wide = slots64 == 256 ? n > 32 && 4 * tiles64 * ksg >= 3 * 256
+                                     : (fold64 || !fold32) && 100ull * tiles32 * k64 >= 92ull * 2 * slots64 * rounds64;
+    p.tok = wide ? 64 : 32;
+    p.fold = wide ? fold64 : fold32;
   }
   return p;
 }
@@ -1279,14 +1283,8 @@ hipError_t pq_dense(const LayerDev& L, const FwdBufs& B, uint32_t n, uint32_t ks
     a.ksg = ksg;
     a.y = B.y;
     const dim3 grid(L.d / pf_rows<QT>(false), (n + p.tok - 1) / p.tok, p.fold ? 1 : ksg);
-    if constexpr (PQ<QT>::SBW == 16) {
-      if (p.tok == 64) {
-        hipLaunchKernelGGL((k_pq<QT, false, 64>), grid, dim3(64 * PF<QT>::NW), 0, st, a);
-        return hipGetLastError();
-      }
-    }
-    if (p.tok != 32) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_pq<QT, false, 32>), grid, dim3(64 * PF<QT>::NW), 0, st, a);
+    if (p.tok == 64) hipLaunchKernelGGL((k_pq<QT, false, 64>), grid, dim3(64 * PF<QT>::NW), 0, st, a);
+    else hipLaunchKernelGGL((k_pq<QT, false, 32>), grid, dim3(64 * PF<QT>::NW), 0, st, a);
     return hipGetLastError();
   }
 }

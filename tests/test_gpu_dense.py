@@ -224,12 +224,14 @@ def test_dense_packed_on_mfma(dev, qtype):
 
 @pytest.mark.parametrize("qtype,rows,cols,ns", [
     # 16 tokens and fewer run the decode kernels, these k_pq in its forms: half-full and ragged tiles
-    # of 32, 64 tokens a workgroup (16-value sub-blocks on full grids), slices of uneven unit ranges,
-    # one slice, one unit a row, the K slices folded in one workgroup
+    # of 32, 64 tokens a workgroup (Q6_K, and full rounds of the others), slices of uneven unit
+    # ranges, one slice, one unit a row, the K slices folded in one workgroup
     (G.Q4_K, 4096, 1792, (17, 33, 250)), (G.Q5_K, 4096, 1024, (20, 64)), (G.Q8_0, 4096, 2304, (23, 130)),
     (G.Q2_K, 4096, 1536, (17, 250)), (G.Q3_K, 4096, 4096, (24, 250)), (G.Q6_K, 4096, 4096, (33, 129)),
     (G.Q4_K, 256, 256, (32, 97)), (G.Q3_K, 768, 512, (41, 300)), (G.Q6_K, 512, 2816, (48, 65)),
-    (G.Q4_K, 256, 1024, (24577,)), (G.Q6_K, 16384, 768, (65, 256)), (G.Q2_K, 8192, 1024, (1025,))])
+    (G.Q4_K, 256, 1024, (24577,)), (G.Q6_K, 16384, 768, (65, 256)), (G.Q2_K, 8192, 1024, (1025,)),
+    (G.Q4_K, 4096, 4096, (250,)), (G.Q8_0, 8192, 4096, (128,)), (G.Q5_K, 2048, 4096, (510,)), (G.Q4_K, 8192, 1024, (1025,)),
+    (G.Q4_K, 4096, 512, (2040,)), (G.Q3_K, 4096, 768, (2048,))])
 def test_dense_packed_rows_do_not_depend_on_the_batch(dev, qtype, rows, cols, ns):
     # a token's row has the same bits in a large batch as in one of at most 16 tokens
     e, _ = O.block_layout(qtype)
