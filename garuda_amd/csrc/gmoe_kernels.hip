@@ -1403,12 +1403,14 @@ static bool prefill_type(uint32_t qt) {
 bool prefill_ok(const LayerDev& L, uint32_t n) {
   const uint32_t nk = n * L.k;
   // rows: gate/up workgroups take up to 256 rows of f, down ones 256 of d (F16: 512). Other
-  // multiples of 256 of d stay on the decode kernels, whose f32 activations have no fp16 pair's range
+  // multiples of 256 of d stay on the decode kernels, which hold the activations in f32: k_pf's
+  // fp16 pairs have less range
   return L.math == 1 && nk >= kPfMinSlots && nk >= 4 * L.ne && L.qt_gate == L.qt_up && prefill_type(L.qt_gate) &&
          prefill_type(L.qt_down) && L.d % 512 == 0 && L.f % 256 == 0 && L.ne < 65536;
 }
 
-// A dense projection run through the down-product path: rows = L.d, width = L.f.
+// A dense projection run through the down-product path: rows = L.d, width = L.f. (L.d: as in
+// prefill_ok.)
 bool prefill_dense_ok(const LayerDev& L, uint32_t n) {
   return L.math == 1 && n >= kPfMinSlots && prefill_type(L.qt_down) && L.d % 512 == 0 && L.f % 256 == 0;
 }
@@ -1518,6 +1520,8 @@ constexpr uint32_t pq_min_per_expert(uint32_t qt) {
 // Q4_K at 48 tokens of the Mixtral shape: 437 us with the int8 down product, 393 with k_pf's.
 bool packed_down_pf(const LayerDev& L, uint32_t n) { return n * L.k >= kPfDownPerExpert * L.ne; }
 
+// (d a multiple of 512: as in prefill_ok, for k_pf's down product; the calls below its line share
+// the rule, untimed at other widths.)
 bool prefill_packed_ok(const LayerDev& L, uint32_t n) {
   const uint32_t nk = n * L.k;
   return L.math == 0 && nk >= kPfMinSlots && nk >= pq_min_per_expert(L.qt_gate) * L.ne && L.qt_gate == L.qt_up &&
