@@ -1217,11 +1217,13 @@ hipError_t pq_gateup(const LayerDev& L, const FwdBufs& B, uint32_t n, hipStream_
     // Three waves a SIMD lose to two where the workgroups, about one token tile an expert up to
     // 20 tokens an expert, take two rounds either way and fill the second of three a CU to a
     // third at most: 8 experts of 14336 rows (896 workgroups), 64 tokens, Q4_K 431 us and 410, Q3_K 539 and 511;
-    // skewed loads 485 and 477, 608 and 593. 128 experts of 768 (768): 219 and 271.
+    // skewed loads 485 and 477, 608 and 593. 128 experts of 768 (768): 219 and 271. Q2_K, whose three
+    // waves spill 16 registers: 128 tokens 731 and 631, 200 tokens 925 and 820 (skewed 996 and 959;
+    // at 112, the most against it, 844 and 935), equal from 256 on.
     bool two = false;
     if constexpr (W == 3) {
       const uint32_t wgs = grid.x * L.ne;
-      two = a.nk <= 20 * L.ne && wgs > 3 * 256 && wgs <= 4 * 256;
+      two = a.nk <= (QT == Q2_K ? 50 : 20) * L.ne && wgs > 3 * 256 && wgs <= 4 * 256;
     }
     if (!B.hh) {
       if constexpr (pq_int8_down(QT)) {

@@ -108,6 +108,7 @@ def test_packed_prefill_at_twelve_an_expert(dev, qts):
 def test_packed_prefill_with_two_workgroups_a_cu(dev):
     # 8 experts of 104 row blocks: 832 workgroups, which run two a CU up to 20 tokens an expert
     check_layer(dev, 512, 13312, 8, 2, (G.Q4_K,) * 3, (36, 64, 80, 81), G.MATH_PACKED, seed=85)
+    check_layer(dev, 512, 13312, 8, 2, (G.Q2_K,) * 3, (200, 201), G.MATH_PACKED, seed=86)
 
 
 @pytest.mark.parametrize("qts", [(G.Q4_K,) * 3, (G.Q3_K, G.Q3_K, G.Q4_K), (G.Q3_K, G.Q3_K, G.Q2_K),
